@@ -113,7 +113,7 @@ def draw(rng):
         return {"kind": kind, "model": rng.choice(sorted(MODELS)), "batch": _log(rng, 1, max(1, min(4, 1024 // seq))),
                 "seq": seq, "start": rng.choice([0, rng.randint(1, 1500)])}
     if kind == "mlp":
-        return {"kind": kind, "model": rng.choice(sorted(MODELS)), "rows": _log(rng, 1, 1024)}
+        return {"kind": kind, "model": rng.choice(sorted(MODELS)), "rows": _log(rng, 1, 768)}
     return {"kind": kind, "rows": _log(rng, 1, 96), "vocab": rng.choice([VOCAB, rng.randint(32000, VOCAB)]),
             "k": rng.choice([1, 20, 40, 64, rng.randint(1, 64)])}
 
