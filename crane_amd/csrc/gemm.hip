@@ -45,7 +45,10 @@
 namespace crane {
 namespace {
 
-constexpr size_t kDefaultWorkspace = 32u << 20;
+// hipBLASLt's stream-K products keep one f32 256 x 256 partial tile per CU:
+// 64 MiB on 256 CUs.
+constexpr size_t kDefaultWorkspace = 64u << 20;
+constexpr int kAlgoCandidates = 16;
 
 // ---------------------------------------------------------------- streaming
 
@@ -694,16 +697,24 @@ class Gemm {
         const uint64_t wsb = ws_bytes_;
         ok = ok && hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &wsb,
                                                          sizeof(wsb)) == HIPBLAS_STATUS_SUCCESS;
-        hipblasLtMatmulHeuristicResult_t res{};
+        hipblasLtMatmulHeuristicResult_t res[kAlgoCandidates] = {};
         int found = 0;
-        ok = ok && hipblasLtMatmulAlgoGetHeuristic(handle_, p.desc, p.a, p.b, p.d, p.d, pref, 1, &res, &found) ==
-                       HIPBLAS_STATUS_SUCCESS;
+        ok = ok && hipblasLtMatmulAlgoGetHeuristic(handle_, p.desc, p.a, p.b, p.d, p.d, pref, kAlgoCandidates, res,
+                                                   &found) == HIPBLAS_STATUS_SUCCESS;
         if (pref) (void)hipblasLtMatmulPreferenceDestroy(pref);
-        if (!ok || found < 1 || res.state != HIPBLAS_STATUS_SUCCESS) {
+        // The first algorithm whose workspace this context holds: the
+        // heuristic also returns algorithms that need more than the
+        // preference's limit (stream-K at M = 1000, N = 37888, K = 3584 asks
+        // for 64 MiB of a 32 MiB limit), and such a product writes past it.
+        int pick = 0;
+        while (ok && pick < found &&
+               (res[pick].state != HIPBLAS_STATUS_SUCCESS || res[pick].workspaceSize > ws_bytes_))
+            ++pick;
+        if (!ok || pick >= found) {
             free_plan(p);
             return CRANE_HIP_E_INVALID;  // no algorithm for this shape / dtype
         }
-        p.algo = res.algo;
+        p.algo = res[pick].algo;
         auto ins = plans_.emplace(key, p);
         *out = &ins.first->second;
         return CRANE_HIP_OK;

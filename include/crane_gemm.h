@@ -48,7 +48,7 @@ extern "C" {
 
 typedef struct crane_gemm crane_gemm;
 
-/* A context with `workspace_bytes` of GEMM workspace (0 for the default, 32 MiB). */
+/* A context with `workspace_bytes` of GEMM workspace (0 for the default, 64 MiB). */
 int crane_gemm_create(size_t workspace_bytes, crane_gemm** out);
 void crane_gemm_destroy(crane_gemm* g);
 

@@ -123,6 +123,38 @@ def test_linear_parity(gpu, orc, dtype, M, N, K, bias):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("workspace", [0, 1 << 20])
+def test_library_product_keeps_to_its_workspace(gpu, workspace):
+    """Qwen2.5-7B gate_up over 1000 token rows: hipBLASLt's first choice needs
+    64 MiB of workspace, whatever limit it was given.  The context takes an
+    algorithm its own workspace holds (the default's 64 MiB, and 1 MiB).
+    Every value lies within an ulp and the f32 accumulation bound of the f32
+    product."""
+    import ctypes
+    import torch
+    from crane_amd import _lib
+    M, N, K = 1000, 37888, 3584
+    print(f"linear with a workspace of {workspace} bytes, M={M} N={N} K={K}", flush=True)
+    gen = torch.Generator(device=gpu).manual_seed(17)
+    x = torch.randn((M, K), generator=gen, device=gpu, dtype=torch.bfloat16)
+    w = torch.randn((N, K), generator=gen, device=gpu, dtype=torch.bfloat16) * K ** -0.5
+    y = torch.empty((M, N), dtype=torch.bfloat16, device=gpu)
+    lib = _lib.lib()
+    h = ctypes.c_void_p()
+    _lib.check(lib.crane_gemm_create(workspace, ctypes.byref(h)), "create")
+    try:
+        _lib.check(lib.crane_gemm_linear(h, x.data_ptr(), w.data_ptr(), None, y.data_ptr(), M, N, K, _lib.BF16,
+                                         torch.cuda.current_stream(gpu).cuda_stream), "linear")
+        torch.cuda.synchronize()
+    finally:
+        lib.crane_gemm_destroy(h)
+    for n0 in range(0, N, 9472):
+        ref = x.float() @ w[n0:n0 + 9472].float().T
+        bound = x.float().abs() @ w[n0:n0 + 9472].float().abs().T * (2 * K * 2.0 ** -24) + ref.abs() * 2.0 ** -8 + 1e-30
+        assert bool(((y[:, n0:n0 + 9472].float() - ref).abs() <= bound).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,bias", [
     (32, 16384, 1152, False),  # the decode batch of config 3; 9 stages of 128
     (17, 16448, 384, True),    # a partial second token group; 3 stages; 257 workgroups
