@@ -14,7 +14,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libcrane_hip.so")
-SOURCES = ["capi.hip", "rope.hip", "append.hip", "decode.hip", "prefill.hip", "kvcache.hip", "pagedkv.hip", "layer.hip", "gemm.hip", "sampling.hip"]
+SOURCES = ["capi.hip", "rope.hip", "append.hip", "decode.hip", "prefill.hip", "kvcache.hip", "pagedkv.hip", "layer.hip", "gemm.hip", "sampling.hip",
+           "tile_rows.hip", "tile_gated.hip", "tile_parts.hip"]
 # bench.py's HBM read-rate probe: a separate library, not part of the C ABI
 PROBE_SRC = os.path.join(CSRC, "probe", "hbm_probe.hip")
 PROBE_LIB = os.path.join(HERE, "libcrane_probe.so")
@@ -46,7 +47,7 @@ def _compile(src: str) -> str:
 
 def build(verbose: bool = True) -> str:
     os.makedirs(BUILD, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=min(4, len(SOURCES))) as ex:
+    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as ex:
         objs = list(ex.map(_compile, SOURCES))
     tmp = LIB + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs, "-lhipblaslt"]

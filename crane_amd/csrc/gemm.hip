@@ -6,30 +6,16 @@
 // B = x viewed as [K, M], D = y viewed as [N, M]; the bias vector (one value
 // per row of D, i.e. per output feature) is the BIAS epilogue.
 //
-// Decode products (bf16, M <= 32 token rows) go to hand-written kernels
-// instead: at M = 32 the product is a stream of W through the chip (2 bytes of
-// W per 2 M flops).  Those whose K is a whole number of the per-wave rings
-// (K <= 8192; the Qwen3-8B decode step's qkv_proj, o_proj, gate_up and
-// lm_head) take the per-wave ring kernel below; other wide ones (N >= 16384)
-// the streaming kernel; the rest, down_proj among them, hipBLASLt.  A
-// product whose output only feeds a residual add (a decode step's o_proj and
-// down_proj) or the fused append (its qkv_proj) can instead leave f32 split-K
-// partial products for the add + norm or the append to sum
-// (crane_gemm_linear_split: the ring kernel's PARTIAL form).  The
-// streaming kernel (measured at the Qwen3-8B decode shapes before the ring
-// kernel: gate_up [24576, 4096] 43 us vs hipBLASLt's 47 us, lm_head
-// [151936, 4096] 241 us vs ~355 us):
-//  - a workgroup of 4 waves owns 64 output features and all of K; wave w
-//    multiplies features 16 w .. 16 w + 15 (the A operand of
-//    v_mfma_f32_16x16x32_bf16) by the token rows (the B operand), f32
-//    accumulation;
-//  - K is streamed in stages of 128: the 64 W rows (256 bytes each) and the
-//    token rows of x are copied HBM -> LDS by bounds-checked buffer_load ...
-//    lds, each 1 KiB copy reading 4 whole 256-byte row pieces (x rows past M
-//    read as zero), into a ring of three stage buffers so two stages are in
-//    flight while one is multiplied;
-//  - 16-byte chunks are XOR-swizzled by row in LDS, so the 16 rows of one
-//    fragment read (ds_read_b128) fall in 16 different bank groups.
+// bf16 products with few token rows go to hand-written kernels instead: the
+// product is then a stream of W through the chip (2 bytes of W per 2 M flops).
+// Up to 32 rows, those whose K is a whole number of the per-wave rings
+// (K <= 8192; a Qwen3-8B decode step's qkv_proj, o_proj and gate_up) take the
+// per-wave ring kernel below; the lm_head and most others up to a few hundred
+// rows take tile_gemm.h's kernel (tile_takes has the line and both sides of
+// it); the rest hipBLASLt.  A product whose output only feeds a residual add (a
+// decode step's o_proj and down_proj) or the fused append (its qkv_proj) can
+// instead leave f32 split-K partial products for the add + norm or the append
+// to sum (crane_gemm_linear_split: the ring kernel's PARTIAL form).
 // Rounding: f32 accumulation, y = bf16(acc + b) (one rounding, as the
 // hipBLASLt bias epilogue).
 #include <hipblaslt/hipblaslt.h>
@@ -39,7 +25,7 @@
 #include <new>
 #include <tuple>
 
-#include "common.h"
+#include "tile_gemm.h"
 #include "../../include/crane_gemm.h"
 
 namespace crane {
@@ -50,175 +36,12 @@ namespace {
 constexpr size_t kDefaultWorkspace = 64u << 20;
 constexpr int kAlgoCandidates = 16;
 
-// ---------------------------------------------------------------- streaming
-
-constexpr int kSkStageK = 128;   // k per pipeline stage (256 bytes of every row)
-constexpr int kSkWaves = 4;      // waves per workgroup; each owns 16 output features
-constexpr int kSkRows = 16 * kSkWaves;
-constexpr int kSkMaxM = 32;      // token rows the streaming kernel takes
+constexpr int kDecodeRows = 32;  // token rows the ring kernel takes
 
 __device__ __forceinline__ bf16x8_v as_bf16x8(uint4 u) { return __builtin_bit_cast(bf16x8_v, u); }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t sk_rsrc(const void* base, uint32_t bytes) {
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
-}
-
-// LDS image of one stage: rows of 256 bytes (16 chunks of 16 bytes, chunk c
-// of row r stored at slot c ^ (r & 15), so the 16 rows one fragment read
-// touches hit 16 different bank groups), W rows first, then x rows.
-template <int MT>
-struct SkStage {
-    static constexpr int kWBytes = kSkRows * 256;
-    static constexpr int kXBytes = 16 * MT * 256;
-    static constexpr int kBytes = kWBytes + kXBytes;
-    static constexpr int kCopies = kBytes / 1024 / kSkWaves;  // 1 KiB copies per wave per stage
-    static_assert(kBytes % (1024 * kSkWaves) == 0, "stage copies split evenly over the waves");
-};
-
-// The voffset of copy i of a wave: copy blk (of the stage's kBytes / 1024)
-// fills LDS bytes [1024 blk, +1024): rows 4 blk + lane / 16 of the stage, slot
-// lane % 16, from chunk slot ^ (row & 15) of that row's 256 bytes.  The stage's
-// k offset is the scalar offset; W rows read from the W resource, x rows
-// (token rows; rows past M read as zero) from the x resource.
-template <int MT>
-__device__ __forceinline__ uint32_t sk_voffset(int blk, int lane, int K) {
-    const int row = 4 * blk + (lane >> 4);
-    const int slot = lane & 15;
-    const int r = row < kSkRows ? row : row - kSkRows;
-    return (uint32_t)r * (uint32_t)K * 2u + 16u * (uint32_t)(slot ^ (r & 15));
-}
-
-// The W resource covers the workgroup's 64 rows (wb, wbytes), the x resource
-// the M token rows (xb, xbytes).
-struct SkSrc {
-    const bf16_t* wb;
-    const bf16_t* xb;
-    uint32_t wbytes, xbytes;
-};
-
-// Issue this wave's copies of one stage into `dst`; soff is the stage's byte
-// offset along k.  (Not a template: the host pass cannot form the LDS pointer
-// the copy takes.)
-__device__ __forceinline__ void sk_issue(uint8_t* dst, const SkSrc& src, const uint32_t* vofs, const bool* isw, int nc,
-                                         int wave, int soff) {
-#pragma unroll
-    for (int i = 0; i < nc; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(isw[i] ? sk_rsrc(src.wb, src.wbytes) : sk_rsrc(src.xb, src.xbytes),
-                                                 dst + (wave * nc + i) * 1024, 16, vofs[i], soff, 0, 0);
-}
-
-// One pipeline stage: wait for stage st (in `cur`), refill `nxt` (the buffer
-// of stage st - 1, which every wave has finished) with stage st + 2, and
-// multiply stage st.
-template <int MT>
-__device__ __forceinline__ void sk_stage(const uint8_t* cur, uint8_t* nxt, int st, int nst, const SkSrc& src,
-                                         const uint32_t (&vofs)[SkStage<MT>::kCopies],
-                                         const bool (&isw)[SkStage<MT>::kCopies], int wave, int wrow, int r, int q,
-                                         f32x4_v (&acc)[MT]) {
-    using St = SkStage<MT>;
-    // this wave's copies of stage st have landed (those of st + 1 may fly),
-    // and its LDS reads of stage st - 1 have completed (lgkmcnt 0: the
-    // compiler may have left the last products of stage st - 1, and their
-    // waits, below this point)
-    if (st + 1 < nst)
-        __builtin_amdgcn_s_waitcnt(0x0070 | (St::kCopies & 15) | ((St::kCopies >> 4) << 14));
-    else
-        __builtin_amdgcn_s_waitcnt(0x0070);
-    // Every wave's copies of stage st have landed and every wave has finished
-    // reading stage st - 1, so the refill below may overwrite it.  A plain
-    // barrier: a release fence here would wait for the copies still in flight
-    // (they count as LDS writes); the acquire fence keeps the reads below it.
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    if (st + 2 < nst) sk_issue(nxt, src, vofs, isw, St::kCopies, wave, (st + 2) * kSkStageK * 2);
-#pragma unroll
-    for (int j = 0; j < kSkStageK / 32; ++j) {
-        const int c = 4 * j + q;
-        const uint4 a = *reinterpret_cast<const uint4*>(cur + wrow * 256 + 16 * (c ^ (wrow & 15)));
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const int t = 16 * m + r;
-            const uint4 bx = *reinterpret_cast<const uint4*>(cur + St::kWBytes + t * 256 + 16 * (c ^ (t & 15)));
-            acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a), as_bf16x8(bx), acc[m], 0, 0, 0);
-        }
-    }
-}
-
-// y = x[M, K] W[N, K]^T (+ b): N / 64 workgroups of 256 threads; workgroup
-// `tile` owns features [64 tile, +64).  Wave w multiplies features 16 w .. +15
-// (the A operand) by the MT token groups of 16 (the B operand).  Lane l holds
-// A row l % 16 / B column l % 16 with the k elements of chunk (4 j + l / 16) of
-// k-step j of a stage; accumulator element i is feature 16 w + 4 (l / 16) + i
-// and token 16 m + l % 16.
-template <int MT>
-__global__ __launch_bounds__(64 * kSkWaves) void skinny_gemm_kernel(const bf16_t* __restrict__ x,
-                                                                    const bf16_t* __restrict__ w,
-                                                                    const bf16_t* __restrict__ bias,
-                                                                    bf16_t* __restrict__ y, int M, int N, int K) {
-    using St = SkStage<MT>;
-    // three stage buffers as separate objects: the compiler's wait-count pass
-    // then knows which buffer each copy writes and waits only for that one
-    __shared__ __attribute__((aligned(1024))) uint8_t lds0[St::kBytes];
-    __shared__ __attribute__((aligned(1024))) uint8_t lds1[St::kBytes];
-    __shared__ __attribute__((aligned(1024))) uint8_t lds2[St::kBytes];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int tile = blockIdx.x;
-    const int nst = K / kSkStageK;
-    const SkSrc src{w + (int64_t)tile * kSkRows * K, x, (uint32_t)kSkRows * K * 2, (uint32_t)M * K * 2};
-    uint32_t vofs[St::kCopies];
-    bool isw[St::kCopies];
-#pragma unroll
-    for (int i = 0; i < St::kCopies; ++i) {
-        const int blk = wave * St::kCopies + i;
-        vofs[i] = sk_voffset<MT>(blk, lane, K);
-        isw[i] = 4 * blk < kSkRows;  // uniform per copy
-    }
-    const int r = lane & 15, q = lane >> 4;
-    const int wrow = 16 * wave + r;
-    f32x4_v acc[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) acc[m] = f32x4_v{};
-    sk_issue(lds0, src, vofs, isw, St::kCopies, wave, 0);
-    if (nst > 1) sk_issue(lds1, src, vofs, isw, St::kCopies, wave, kSkStageK * 2);
-    // stage st lives in buffer st % 3; the loop is unrolled by three so every
-    // access names its buffer
-    for (int st = 0; st < nst; st += 3) {
-        sk_stage<MT>(lds0, lds2, st, nst, src, vofs, isw, wave, wrow, r, q, acc);
-        if (st + 1 < nst) sk_stage<MT>(lds1, lds0, st + 1, nst, src, vofs, isw, wave, wrow, r, q, acc);
-        if (st + 2 < nst) sk_stage<MT>(lds2, lds1, st + 2, nst, src, vofs, isw, wave, wrow, r, q, acc);
-    }
-    const int n = tile * kSkRows + 16 * wave + 4 * q;
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const int t = 16 * m + r;
-        if (t >= M) continue;
-        float v[4] = {acc[m][0], acc[m][1], acc[m][2], acc[m][3]};
-        if (bias) {
-            float bv[4];
-            load4(bias + n, bv);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] += bv[e];
-        }
-        store4(y + (int64_t)t * N + n, v);
-    }
-}
-
-// The streaming kernel takes bf16 products with few token rows and enough
-// output features for 256 workgroups (one per CU); K in whole stages, and
-// buffer offsets of the 64 W rows and of x within 32 bits.
-bool skinny_fits(int64_t M, int64_t N, int64_t K) {
-    return M >= 1 && M <= kSkMaxM && N % kSkRows == 0 && N / kSkRows >= 256 && N <= 0x7fffffff &&
-           K % kSkStageK == 0 && (int64_t)kSkRows * K * 2 <= 0xffffffffLL && M * K * 2 <= 0xffffffffLL;
-}
-
-int launch_skinny(const bf16_t* x, const bf16_t* w, const bf16_t* bias, bf16_t* y, int M, int N, int K,
-                  hipStream_t st) {
-    const dim3 grid((unsigned)(N / kSkRows)), block(64 * kSkWaves);
-    if (M <= 16)
-        hipLaunchKernelGGL((skinny_gemm_kernel<1>), grid, block, 0, st, x, w, bias, y, M, N, K);
-    else
-        hipLaunchKernelGGL((skinny_gemm_kernel<2>), grid, block, 0, st, x, w, bias, y, M, N, K);
-    return launch_status(hipGetLastError());
 }
 
 // ---------------------------------------------------------------- per-wave rings
@@ -233,8 +56,7 @@ int launch_skinny(const bf16_t* x, const bf16_t* w, const bf16_t* bias, bf16_t* 
 // and wave 0 adds them in wave order (fixed, so a call's bits repeat).
 // Measured at the Qwen3-8B decode shapes (32 rows, weights rotated past the
 // Infinity Cache): o_proj [4096, 4096] 11.4 us against hipBLASLt's 13.8,
-// qkv_proj [6144, 4096] 13.5 against 15.8, gate_up [24576, 4096] 31.8 against
-// the streaming kernel's 43.0, lm_head [151936, 4096] 221 against 238.  The x
+// qkv_proj [6144, 4096] 13.5 against 15.8, gate_up [24576, 4096] 31.8.  The x
 // reads are what bounds it: without them the same kernel streams W at 5.2-6.0
 // TB/s, and x (the same bytes for every workgroup, read from L2) grows with
 // 32 token rows / 16 FT features per W byte, so wider workgroups pay less x
@@ -340,8 +162,8 @@ __global__ __launch_bounds__(64 * KS) void ring_gemm_kernel(const bf16_t* __rest
     // The W resources span the workgroup's rows from this wave's k0: its 16 H
     // rows (GATED: the gate rows, and the up rows N / 2 further).
     const int64_t row0 = (int64_t)tile * 16 * H;
-    const __amdgpu_buffer_rsrc_t src_lo = sk_rsrc(w + row0 * K + k0, (uint32_t)16 * H * K * 2);
-    const __amdgpu_buffer_rsrc_t src_hi = sk_rsrc(w + (row0 + (GATED ? N / 2 : 0)) * K + k0, (uint32_t)16 * H * K * 2);
+    const __amdgpu_buffer_rsrc_t src_lo = row_rsrc(w + row0 * K + k0, (uint32_t)16 * H * K * 2);
+    const __amdgpu_buffer_rsrc_t src_hi = row_rsrc(w + (row0 + (GATED ? N / 2 : 0)) * K + k0, (uint32_t)16 * H * K * 2);
     uint32_t vofs[4 * H];
 #pragma unroll
     for (int c = 0; c < 4 * H; ++c) {
@@ -482,7 +304,7 @@ struct RingCfg {
 constexpr int kRingCUs = 256;
 
 RingCfg ring_cfg(int64_t M, int64_t N, int64_t K, bool gated = false) {
-    if (M < 1 || M > kSkMaxM || K < 1 || K > kRingMaxK || N < 1 || N > 0x7fffffff) return {0, 0, 0};
+    if (M < 1 || M > kDecodeRows || K < 1 || K > kRingMaxK || N < 1 || N > 0x7fffffff) return {0, 0, 0};
     RingCfg c{0, 0, 0};
     if (N > 8192) {
         int64_t best = 0;
@@ -545,7 +367,7 @@ int launch_ring(const RingCfg& c, const bf16_t* x, const bf16_t* w, const bf16_t
 // 4), down_proj [4096 x 12288] in 4 splits 19.3 -> 18.4 us (1 wave and a ring
 // of 3 against 2 waves).  {0, 0, 0} when the shape does not split this way.
 RingCfg split_cfg(int64_t M, int64_t N, int64_t K, int64_t splits) {
-    if (M < 1 || M > kSkMaxM || N < 32 || N > 0x7fffffff || K < 1 || splits < 2 || splits > 16 || K % splits)
+    if (M < 1 || M > kDecodeRows || N < 32 || N > 0x7fffffff || K < 1 || splits < 2 || splits > 16 || K % splits)
         return {0, 0, 0};
     const int64_t kp = K / splits;
     if (kp > 32768) return {0, 0, 0};
@@ -592,6 +414,88 @@ void launch_split(const RingCfg& c, const bf16_t* x, const bf16_t* w, float* par
         launch_split_ft<MT, 2, 2>(c.ft, grid, x, w, part, M, N, K, st);
 }
 
+// ---------------------------------------------------------------- tiles
+//
+// Which bf16 products take tile_gemm.h's kernel (after the ring kernel), both
+// sides measured over the Qwen3-0.6B, Qwen3-8B and Qwen2.5-7B projections at
+// 1 to 300 rows, weights read from HBM, hipBLASLt first:
+//   M <= 32:   where the library reads W slowly: gate_up pairs (63.4 -> 44.2
+//              us at [37888 x 3584]); wide N (lm_head [151936 x 4096] at 32
+//              rows 222 (ring kernel) -> 200); K > 8192 ([3584 x 18944] 105
+//              -> 27.6); small weights ([1024 x 3072] 10.1 -> 7.7).  Elsewhere
+//              ([4608 x 3584] at 20 rows: 11.6 against 12.8) the library;
+//   M <= 128:  all (1.36 times as fast in the geometric mean; the closest,
+//              [1024 x 3072] at 96 rows, 8.6 -> 8.8) but gate_up pairs wider
+//              than 32768 past 96 rows (74 -> 81);
+//   M <= 224:  N <= 8192 ([4096 x 4096] at 200 rows 21.9 -> 16.6; gate_up
+//              [24576 x 4096] at 160: 58.9 -> 65.3, so wide N stays);
+//   M <= 320:  N <= 8192 and N K <= 20 M ([4608 x 3584] at 256 rows 34.6 ->
+//              21.4, [4096 x 12288] 55.0 -> 57.5).
+constexpr int64_t kTileWideN = 32768;
+
+bool tile_takes(int64_t M, int64_t N, int64_t K, bool gated) {
+    if (M < 1 || K < 64 || K % 64 || K > (1 << 20) || N < 8 || N % (gated ? 16 : 8) || N > 0x7fffffff) return false;
+    const int64_t nk = N * K;
+    if (M <= kDecodeRows) return gated || N > 8192 || K > 8192 || nk <= (8 << 20);
+    if (M <= 128) return !gated || N <= kTileWideN || M <= 96;
+    return N <= 8192 && (M <= 224 || (M <= 320 && nk <= 20000000));
+}
+
+// The form with the least time by a fit to the same sweep (2% over the best
+// form in the mean): with `per` workgroups on the busiest of 256 CUs and
+// `stages` of 64 k each, per stages (0.036 FT + 0.027 MT + 0.017 FT MT) us (its
+// copies and products) + 0.29 per, and for splits the sums' extra launch and
+// bytes.  4 token tiles only where they cover M (their second block measured
+// slower than 3), 160 features only for gate_up pairs in one round of
+// workgroups ([37888 x 3584]: 237 of them).
+TileCfg tile_cfg(int64_t M, int64_t N, int64_t K, bool gated, size_t ws_bytes) {
+    TileCfg best{0, 0, 0};
+    double least = 0;
+    for (int splits = 1; splits <= (gated ? 1 : 8); splits *= 2) {
+        if (K % (64 * splits) || (splits > 1 && (size_t)M * N * splits * 4 > ws_bytes)) continue;
+        for (int ft = 1; ft <= (gated ? 5 : 4); ++ft)
+            for (int mt = 1; mt <= (ft < 4 ? 4 : 3); ++mt) {
+                const int64_t tb = (M + 32 * mt - 1) / (32 * mt);
+                if ((tb > 1 && mt == 4) || 32 * mt >= M + 32) continue;
+                const int64_t per_tile = (gated ? 16 : 32) * ft, nout = gated ? N / 2 : N;
+                const int64_t wgs = (nout + per_tile - 1) / per_tile * tb * splits;
+                const int64_t per = (wgs + 255) / 256;
+                if (ft == 5 && per > 1) continue;
+                double t = per * (K / 64.0 / splits * (0.0355 * ft + 0.0266 * mt + 0.0165 * ft * mt) + 0.29);
+                if (splits > 1) t += 2.6 + 0.65e-6 * (double)(M * N * splits * 4);
+                if (!best.ft || t < least) best = TileCfg{ft, mt, splits}, least = t;
+            }
+    }
+    return best;
+}
+
+// y = bf16(sum over splits of parts + bias), 8 features a thread: 32-bit sums
+// in split order, one rounding.  grid (ceil(N / 8 / 256), M).
+template <int NP>
+__global__ __launch_bounds__(256) void sum_parts_kernel(const float* __restrict__ parts,
+                                                        const bf16_t* __restrict__ bias, bf16_t* __restrict__ y, int M,
+                                                        int N) {
+    const int n = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 8;
+    if (n >= N) return;
+    const int64_t at = (int64_t)blockIdx.y * N + n, plane = (int64_t)M * N;
+    float v[NP][8], b[8];
+#pragma unroll
+    for (int s = 0; s < NP; ++s) load8(parts + s * plane + at, v[s]);
+    if (bias) {
+        load8(bias + n, b);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) b[e] = 0.f;
+    }
+#pragma unroll
+    for (int s = 1; s < NP; ++s)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[0][e] += v[s][e];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[0][e] += b[e];
+    store8(y + at, v[0]);
+}
+
 struct Plan {
     hipblasLtMatmulDesc_t desc = nullptr;
     hipblasLtMatrixLayout_t a = nullptr, b = nullptr, d = nullptr;
@@ -635,14 +539,14 @@ class Gemm {
                hipStream_t st) {
         std::lock_guard<std::mutex> lock(mu_);
         if (dtype == CRANE_HIP_BF16) {
-            const RingCfg rc = ring_cfg(M, N, K);
+            const RingCfg rc = N <= kTileWideN ? ring_cfg(M, N, K) : RingCfg{0, 0, 0};
             if (rc.ft)
                 return launch_ring<false>(rc, (const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)y,
                                           (int)M, (int)N, (int)K, st);
+            if (tile_takes(M, N, K, false))
+                return linear_tile((const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)y, (int)M, (int)N,
+                                   (int)K, st);
         }
-        if (dtype == CRANE_HIP_BF16 && skinny_fits(M, N, K))
-            return launch_skinny((const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)y, (int)M, (int)N,
-                                 (int)K, st);
         Plan* p = nullptr;
         int rc = plan(M, N, K, dtype, bias != nullptr, &p);
         if (rc) return rc;
@@ -665,6 +569,25 @@ class Gemm {
     }
 
   private:
+    // y = x W^T (+ b) by tile_gemm.h's kernel; with splits of K, their sums go
+    // through the context's workspace.
+    int linear_tile(const bf16_t* x, const bf16_t* w, const bf16_t* bias, bf16_t* y, int M, int N, int K,
+                    hipStream_t st) {
+        const TileCfg c = tile_cfg(M, N, K, false, ws_bytes_);
+        TileArgs a{x, w, bias, y, (float*)ws_, M, N, K};
+        const bool ok = c.splits == 1 ? launch_tile_rows(c, a, st) : launch_tile_parts(c, a, st);
+        if (!ok) return CRANE_HIP_E_LAUNCH;
+        if (c.splits > 1) {
+            const dim3 grid((unsigned)((N / 8 + 255) / 256), (unsigned)M);
+#define CRANE_SUM_CASE(n)                                                                                            \
+    if (c.splits == n)                                                                                               \
+        hipLaunchKernelGGL((sum_parts_kernel<n>), grid, dim3(256), 0, st, (const float*)ws_, bias, y, M, N);
+            CRANE_SUM_CASE(2) CRANE_SUM_CASE(4) CRANE_SUM_CASE(8)
+#undef CRANE_SUM_CASE
+        }
+        return launch_status(hipGetLastError());
+    }
+
     // The descriptors and the heuristic's algorithm for one shape, built once.
     int plan(int64_t M, int64_t N, int64_t K, int dtype, bool has_bias, Plan** out) {
         const auto key = std::make_tuple(M, N, K, dtype, has_bias);
@@ -778,6 +701,27 @@ extern "C" int crane_gemm_linear_silu_mul(crane_gemm* g, const void* x, const vo
     if (!crane::aligned16(x) || !crane::aligned16(w) || !crane::aligned16(out)) return CRANE_HIP_E_ALIGN;
     if (!crane_gemm_silu_mul_supported(M, inter, K, dtype)) return CRANE_HIP_E_INVALID;
     return g->impl.linear_silu_mul(x, w, out, M, inter, K, (hipStream_t)stream);
+}
+
+extern "C" int crane_gemm_tile_silu_mul_supported(int64_t M, int64_t inter, int64_t K, int dtype) {
+    if (dtype != CRANE_HIP_BF16 || inter <= 0 || inter > 0x3fffffffLL || inter % 8) return 0;
+    return crane::tile_takes(M, 2 * inter, K, true);
+}
+
+extern "C" int crane_gemm_tile_silu_mul(const void* x, const void* w, void* out, int64_t M, int64_t inter, int64_t K,
+                                        int dtype, void* stream) {
+    if (dtype != CRANE_HIP_F32 && dtype != CRANE_HIP_BF16) return CRANE_HIP_E_DTYPE;
+    if (M < 0 || inter <= 0 || K <= 0 || M > 0x7fffffffLL || inter > 0x3fffffffLL || K > 0x7fffffffLL)
+        return CRANE_HIP_E_INVALID;
+    if (M == 0) return CRANE_HIP_OK;
+    if (!x || !w || !out) return CRANE_HIP_E_INVALID;
+    if (!crane::aligned16(x) || !crane::aligned16(w) || !crane::aligned16(out)) return CRANE_HIP_E_ALIGN;
+    if (!crane_gemm_tile_silu_mul_supported(M, inter, K, dtype)) return CRANE_HIP_E_INVALID;
+    const crane::TileCfg c = crane::tile_cfg(M, 2 * inter, K, true, 0);
+    const crane::TileArgs a{(const crane::bf16_t*)x, (const crane::bf16_t*)w, nullptr, (crane::bf16_t*)out, nullptr,
+                            (int)M, (int)(2 * inter), (int)K};
+    if (!crane::launch_tile_gated(c, a, (hipStream_t)stream)) return CRANE_HIP_E_LAUNCH;
+    return crane::launch_status(hipGetLastError());
 }
 
 extern "C" int crane_gemm_split_supported(int64_t M, int64_t N, int64_t K, int splits, int dtype) {

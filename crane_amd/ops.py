@@ -676,9 +676,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
 def linear_silu_mul(x: torch.Tensor, gate_up: torch.Tensor) -> torch.Tensor:
     """Crane's Mlp gate / up projections and fused_silu_mul: x [..., K] with
     the merged weight gate_up [2 I, K] (gate rows first) -> silu(gate) * up
-    [..., I].  One launch where the library's gated kernel takes the shape
-    (decode batches, crane_gemm_silu_mul_supported), else linear then
-    silu_mul; the roundings are the same either way."""
+    [..., I].  One launch where one of the library's gated kernels takes the
+    shape (decode batches and short prompts: crane_gemm_silu_mul_supported,
+    crane_gemm_tile_silu_mul_supported), else linear then silu_mul; the
+    roundings are the same either way."""
     dev = _dev(x, gate_up)
     K = x.shape[-1]
     if gate_up.dim() != 2 or gate_up.shape[1] != K or gate_up.shape[0] % 2:
@@ -686,15 +687,21 @@ def linear_silu_mul(x: torch.Tensor, gate_up: torch.Tensor) -> torch.Tensor:
     inter = gate_up.shape[0] // 2
     M = x.numel() // K
     dt = _dtype_code(x)
-    if not _lib.lib().crane_gemm_silu_mul_supported(M, inter, K, dt):
+    lib = _lib.lib()
+    ring = lib.crane_gemm_silu_mul_supported(M, inter, K, dt)
+    if not ring and not lib.crane_gemm_tile_silu_mul_supported(M, inter, K, dt):
         return silu_mul(linear(x, gate_up), inter)
     _contig(x, "x")
     _contig(gate_up, "gate_up")
     if gate_up.dtype != x.dtype:
         raise CraneHipError(_lib.E_DTYPE, f"gate_up dtype {gate_up.dtype} != {x.dtype}")
     out = torch.empty(x.shape[:-1] + (inter,), dtype=x.dtype, device=dev)
-    check(_lib.lib().crane_gemm_linear_silu_mul(_gemm(dev)._h, x.data_ptr(), gate_up.data_ptr(), out.data_ptr(), M,
-                                                inter, K, dt, _stream(dev)), "linear_silu_mul")
+    if ring:
+        check(lib.crane_gemm_linear_silu_mul(_gemm(dev)._h, x.data_ptr(), gate_up.data_ptr(), out.data_ptr(), M, inter,
+                                             K, dt, _stream(dev)), "linear_silu_mul")
+    else:
+        check(lib.crane_gemm_tile_silu_mul(x.data_ptr(), gate_up.data_ptr(), out.data_ptr(), M, inter, K, dt,
+                                           _stream(dev)), "linear_silu_mul")
     return out
 
 

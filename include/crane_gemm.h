@@ -13,9 +13,10 @@
  * The same call serves the MLP projections (gate_up, down) and the lm_head.
  * Products go to hipBLASLt with f32 accumulation, the bias added in the
  * epilogue (one rounding of acc + b, where candle rounds the product and then
- * the sum), except bf16 products with few token rows (M <= 32), which
- * hand-written kernels run with the same accumulation and rounding: a per-wave
- * ring kernel when K <= 8192 splits into its pipelines, by these rules:
+ * the sum), except bf16 products with few token rows, which hand-written
+ * kernels run with the same accumulation and rounding.  Up to 32 rows and
+ * N = 32768: a per-wave ring kernel when K <= 8192 splits into its pipelines,
+ * by these rules:
  *   N <= 4096:         N a multiple of 16 and K of 2048;
  *   4096 < N <= 8192:  N a multiple of 32 and K of 1024;
  *   N > 8192:          of the configurations of 96 features (K a multiple of
@@ -24,8 +25,14 @@
  *                      busiest CU the fewest features (the first listed on a
  *                      tie); gate_up + SiLU (crane_gemm_linear_silu_mul) takes
  *                      96 or 64 only
- * (the decode step's qkv_proj, o_proj, gate_up and lm_head), else a streaming
- * kernel for N >= 16384 (N a multiple of 64, K of 128).  The kernel that runs
+ * (the decode step's qkv_proj, o_proj, gate_up).  Else an LDS-tile kernel for N
+ * a multiple of 8 and K of 64:
+ *   M <= 32:   N > 8192, K > 8192 or N K <= 8 Mi;
+ *   M <= 128:  every such N and K;
+ *   M <= 224:  N <= 8192;
+ *   M <= 320:  N <= 8192 and N K <= 20 M;
+ * it may split K and sum the splits' f32 products through the context's
+ * workspace.  The kernel that runs
  * a shape fixes the f32 summation order of its products.  A crane_gemm
  * context holds the hipBLASLt handle,
  * a workspace allocated at creation and the algorithm chosen for each shape
@@ -76,6 +83,18 @@ int crane_gemm_silu_mul_supported(int64_t M, int64_t inter, int64_t K, int dtype
  * CRANE_HIP_E_INVALID for a shape crane_gemm_silu_mul_supported rejects. */
 int crane_gemm_linear_silu_mul(crane_gemm* g, const void* x, const void* w, void* out, int64_t M, int64_t inter,
                                int64_t K, int dtype, void* stream);
+
+/* The same product on the LDS-tile kernel, for shapes
+ * crane_gemm_silu_mul_supported rejects: 1 when crane_gemm_tile_silu_mul takes
+ * the shape, else 0: bf16, inter a multiple of 8, K a multiple of 64 up to 2^20,
+ * and M <= 96 rows, or M <= 128 with inter <= 16384, or M <= 224 with
+ * inter <= 4096, or M <= 320 with inter <= 4096 and 2 inter K <= 20 M. */
+int crane_gemm_tile_silu_mul_supported(int64_t M, int64_t inter, int64_t K, int dtype);
+
+/* crane_gemm_linear_silu_mul's product, roundings and layout (its f32
+ * summation order is the kernel's own); no context and no workspace. */
+int crane_gemm_tile_silu_mul(const void* x, const void* w, void* out, int64_t M, int64_t inter, int64_t K, int dtype,
+                             void* stream);
 
 /* 1 when crane_gemm_linear_split takes the shape, else 0: bf16, M <= 32 token
  * rows, N a multiple of 32 or 48, 2 <= splits <= 16, and K a multiple of splits

@@ -207,6 +207,34 @@ def test_linear_ring_parity(gpu, orc, M, N, K, bias):
     assert bool((got == got2).all())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,bias", [
+    (33, 4096, 64, True),      # one stage; a second token tile of one row
+    (40, 1000, 448, True),     # N a multiple of 8 only: a last tile of 8 features; 7 stages, ring of 6
+    (64, 200, 4096, False),    # few features: 8 splits of K, two whole token tiles
+    (77, 2056, 1024, True),    # 4 splits and the bias in their sum; 13 rows of the last token tile
+    (97, 512, 2048, False),    # 4 token tiles over one block of rows
+    (129, 4096, 640, True),    # two blocks of token rows, the second of one row
+    (224, 1024, 3072, False),  # the last row count at any K
+    (320, 2048, 1024, True),   # the last row count of the kernel
+    (321, 2048, 1024, True),   # ... and the library's first
+    (1, 32776, 192, True),     # one row, N past the ring kernel's: 3 stages, a last tile of 8 features
+    (20, 1024, 3072, False),   # a decode batch over a small weight, split
+    (32, 512, 8256, True),     # K past the ring kernel's limit, 129 stages: no even split
+])
+def test_linear_tile_parity(gpu, orc, M, N, K, bias):
+    """bf16 products on the LDS-tile kernel, at the edges of its tiles, rings,
+    splits and row limits; same bar as the library path, and a second call
+    repeats the bits (fixed summation order)."""
+    from crane_amd import ops
+    print(f"linear (tile) M={M} N={N} K={K} bias={bias}", flush=True)
+    x, w, b = _case(2100 + M + N + K, M, N, K, "bf16", bias)
+    got = ops.linear(_t(x, "bf16", gpu), _t(w, "bf16", gpu), _t(b, "bf16", gpu) if bias else None)
+    assert_linear_close(got.float().cpu().numpy(), x, w, b, "bf16", orc, f"tile linear {M}x{N}x{K}")
+    got2 = ops.linear(_t(x, "bf16", gpu), _t(w, "bf16", gpu), _t(b, "bf16", gpu) if bias else None)
+    assert bool((got == got2).all())
+
+
 def test_split_shape_query():
     """Which shapes the split-K partial products take (host logic, no GPU):
     bf16, at most 32 token rows, N a multiple of 32 or 48, K a multiple of the
@@ -286,6 +314,30 @@ def _silu_mul_bound(x, w, orc):
     ref = orc.silu_mul(gu, False, "bf16")
     bound = 1.1 * np.abs(u) * dgu[:, :inter] + np.abs(silu) * dgu[:, inter:] + 2 * bf16_ulp(ref)
     return ref, bound
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,inter,K", [
+    (1, 40, 64),        # one stage; a last tile of 8 outputs
+    (32, 3072, 1024),   # narrow: past the ring kernel's gated shapes
+    (33, 18944, 256),   # 80 outputs a workgroup in one round
+    (77, 6144, 512),    # three token tiles
+    (97, 1032, 448),    # four token tiles; 8 outputs in the last tile
+    (300, 2048, 576),   # three blocks of token rows
+])
+def test_linear_silu_mul_tile_parity(gpu, orc, M, inter, K):
+    """crane_gemm_tile_silu_mul against the oracle chain within the bound of
+    its roundings, bit-repeatable."""
+    from crane_amd import _lib, ops
+    assert _lib.lib().crane_gemm_silu_mul_supported(M, inter, K, _lib.BF16) == 0
+    assert _lib.lib().crane_gemm_tile_silu_mul_supported(M, inter, K, _lib.BF16) == 1
+    print(f"silu_mul (tile) M={M} inter={inter} K={K}", flush=True)
+    x, w, _ = _case(2500 + M + inter + K, M, 2 * inter, K, "bf16", False)
+    ref, bound = _silu_mul_bound(x, w, orc)
+    xd, wd = _t(x, "bf16", gpu), _t(w, "bf16", gpu)
+    got = ops.linear_silu_mul(xd, wd)
+    assert np.all(np.abs(got.float().cpu().numpy().astype(np.float64) - ref) <= bound)
+    assert bool((got == ops.linear_silu_mul(xd, wd)).all())
 
 
 @pytest.mark.gpu
