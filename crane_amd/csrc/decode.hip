@@ -27,8 +27,8 @@
 //      of consecutive keys.
 //   C. P @ V: 16 lanes read a V row (8 dims each); two consecutive rows are
 //      interleaved with v_perm so v_dot2_f32_bf16 takes (p_j, p_j+1) x
-//      (v_j, v_j+1) per dim.  The 4 row groups of a wave are summed with lane
-//      permutes and the 4 waves through LDS.
+//      (v_j, v_j+1) per dim.  The 4 row groups of a wave are summed with row
+//      swaps and the 4 waves through LDS.
 // A sequence that fits one chunk is normalised and written directly; longer
 // ones leave a partial row and its (m, l) in the workspace: for bf16 the row
 // normalised by the chunk's sum l and stored in bf16 (half the bytes the
@@ -67,10 +67,27 @@ constexpr int kMaxSplits = 4096;  // chunks per sequence the merge handles
 constexpr int kKRows = 4;         // K rows in flight per lane in phase A (of 8)
 constexpr int kMaxGroup = 8;    // q heads handled per workgroup
 
-// Sum over the 4 rows (16-lane groups) of the wave; every lane gets the total.
-__device__ __forceinline__ float rows4_sum(float x) {
-    x += __shfl_xor(x, 16);
-    return x + __shfl_xor(x, 32);
+// Sums over the 4 rows (16-lane groups) of the wave of four values at once:
+// row g gets the total of v[g], associated (row 0 + row 1) + (row 2 + row 3).
+// A row swap and an add reduce two values together (v_permlane16_swap_b32
+// exchanges the odd rows of one register with the even rows of another,
+// v_permlane32_swap_b32 the upper half of one with the lower half of the other), so
+// four totals cost 3 swaps and 3 adds where lane permutes through LDS cost 8 of
+// each.  The permutes were the longest serial stretch of a workgroup's tail
+// (16 values per 2 heads, 2 permutes each): chunk + merge, same bits, one
+// sequence of 4000 keys at 32 / 8 heads 9.33 -> 8.51 us, 16 sequences of 500 to
+// 1000 keys at 28 / 4 heads 12.60 -> 11.30, 32 of 500 to 1000 at 32 / 8 22.28 ->
+// 20.48, the ragged batch of 512 to 4096 keys 55.9 -> 55.0.
+__device__ __forceinline__ float swap_add16(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float swap_add32(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float rows4_sum4(float a, float b, float c, float d) {
+    return swap_add32(swap_add16(a, b), swap_add16(c, d));
 }
 
 __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
@@ -375,18 +392,12 @@ __device__ __forceinline__ void decode_item(
         }
     }
     // Sum the 4 row groups of the wave, then the 4 waves through LDS.
+    // (row group g ends up with dims 8 l16 + g and 8 l16 + 4 + g.)
 #pragma unroll
     for (int h = 0; h < G; ++h)
 #pragma unroll
-        for (int d = 0; d < 8; ++d) o[h][d] = rows4_sum(o[h][d]);
-    if (grp == 0) {
-#pragma unroll
-        for (int h = 0; h < G; ++h)
-#pragma unroll
-            for (int d = 0; d < 8; d += 4)
-                *reinterpret_cast<float4*>(&red[wave][h][8 * l16 + d]) =
-                    make_float4(o[h][d], o[h][d + 1], o[h][d + 2], o[h][d + 3]);
-    }
+        for (int d = 0; d < 8; d += 4)
+            red[wave][h][8 * l16 + d + grp] = rows4_sum4(o[h][d], o[h][d + 1], o[h][d + 2], o[h][d + 3]);
     __syncthreads();
 
     for (int e = tid; e < G * kHeadDim; e += kThreads) {
