@@ -1,7 +1,8 @@
 """ctypes binding of libcrane_hip.so, the C ABI declared in include/crane_hip.h
 (attention launchers, dense and paged), include/crane_layer.h (the decoder
 layer's row kernels), include/crane_gemm.h (the QKV / o_proj projections), include/crane_sampling.h
-(argmax, top-k), include/crane_kv.h (host-side KV-cache manager) and
+(argmax, top-k), include/crane_few.h (a decode step's projections at one
+sequence), include/crane_kv.h (host-side KV-cache manager) and
 include/crane_pkv.h (paged KV-cache manager).
 
 The library is the only compute path: there is no CPU fallback.  Loading
@@ -93,6 +94,10 @@ SIGNATURES = {
     "crane_gemm_tile_silu_mul": ([_vp, _vp, _vp, _i64, _i64, _i64, _i, _vp], _i),
     "crane_gemm_split_supported": ([_i64, _i64, _i64, _i, _i], _i),
     "crane_gemm_linear_split": ([_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i, _i, _vp], _i),
+    # include/crane_few.h
+    "crane_few_supported": ([_i64, _i64, _i64, _i, _i, _i], _i),
+    "crane_few_linear": ([_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i, _vp], _i),
+    "crane_few_norm_linear": ([_vp, _vp, _vp, _vp, _f, _vp, _vp, _vp, _i64, _i64, _i64, _i, _i, _vp], _i),
     # include/crane_pkv.h
     "crane_pkv_create": ([_i, _i, _i, _i, _i64, _i, _i, _vpp], _i),
     "crane_pkv_destroy": ([_vp], None),

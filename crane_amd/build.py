@@ -15,7 +15,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libcrane_hip.so")
 SOURCES = ["capi.hip", "rope.hip", "append.hip", "decode.hip", "prefill.hip", "kvcache.hip", "pagedkv.hip", "layer.hip", "gemm.hip", "sampling.hip",
-           "tile_rows.hip", "tile_gated.hip", "tile_parts.hip"]
+           "tile_rows.hip", "tile_gated.hip", "tile_parts.hip", "few_rows.hip"]
 # bench.py's HBM read-rate probe: a separate library, not part of the C ABI
 PROBE_SRC = os.path.join(CSRC, "probe", "hbm_probe.hip")
 PROBE_LIB = os.path.join(HERE, "libcrane_probe.so")

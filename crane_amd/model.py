@@ -96,6 +96,11 @@ class DecoderModel:
         self.scale = 1.0 / math.sqrt(D)
         self.workspace = torch.empty(ops.decode_workspace_bytes(batch, Hq, Hkv, capacity, self.dtype),
                                      dtype=torch.uint8, device=self.device)
+        # one sequence: a decode step's norms run inside its projections
+        self.few = all(ops.few_rows_supported(batch, w.qkv, True) and ops.few_rows_supported(batch, w.o) and
+                       ops.few_rows_supported(batch, w.gate_up, True, True) and
+                       ops.few_rows_supported(batch, w.down) and w.input_norm is not None and
+                       w.post_norm is not None for w in layers)
 
     def shared(self, i: int) -> bool:
         """Layer i reuses its anchor's K/V (Hunyuan CLA)."""
@@ -121,34 +126,47 @@ class DecoderModel:
         to add (fused with the next norm)."""
         cfg, w = self.cfg, self.layers[i]
         B = self.batch
-        D, Hq, Hkv = ops.HEAD_DIM, cfg.num_heads, cfg.num_kv_heads
+        D, Hq = ops.HEAD_DIM, cfg.num_heads
         eps = cfg.rms_norm_eps
-        a = self.anchor(i)
-        if self.shared(i):
-            q = ops.linear(h, w.qkv, w.qkv_bias).view(B, S, Hq * D)
-            q = ops.q_norm_rope(q, self.cos, self.sin, positions, Hq, w.q_norm, eps, self.order)
-        else:
-            # a decode step's qkv_proj goes to the append as split-K partial
-            # products (ops.linear_for_append), reduced inside the append
-            if S == 1:
-                qkv = ops.linear_for_append(h, w.qkv, w.qkv_bias)
-                if not isinstance(qkv, ops.PartialProduct):
-                    qkv = qkv.view(B, S, -1)
-            else:
-                qkv = ops.linear(h, w.qkv, w.qkv_bias).view(B, S, -1)
-            q = ops.qk_norm_rope_append(qkv, self.cos, self.sin, positions, self.k[a], self.v[a], self.lengths,
-                                        bound, Hq, Hkv, w.q_norm, w.k_norm, eps, self.order)
-        if S == 1:
-            attn = ops.attention_decode(q.view(B, Hq, D), self.k[a], self.v[a], lengths_after, bound, self.scale,
-                                        self.workspace, self.score_mode)
-        else:
-            attn = ops.attention_prefill(q, self.k[a], self.v[a], self.lengths, start_bound, self.scale, True)
+        # a decode step's qkv_proj goes to the append as split-K partial
+        # products (ops.linear_for_append), reduced inside the append
+        qkv = (ops.linear_for_append if S == 1 and not self.shared(i) else ops.linear)(h, w.qkv, w.qkv_bias)
+        attn = self._attention(i, qkv if isinstance(qkv, ops.PartialProduct) else qkv.view(B, S, -1), positions,
+                               lengths_after, S, bound, start_bound)
         # In a decode step o_proj and down_proj feed only the adds: their split-K
         # partial products go straight into add_rms_norm (ops.linear_for_residual).
         proj = ops.linear_for_residual if S == 1 else ops.linear
         o = proj(attn.view(B * S, Hq * D), w.o)
         h2 = ops.add_rms_norm(residual, o, w.post_norm, eps)
         return proj(ops.linear_silu_mul(h2, w.gate_up), w.down)
+
+    def _attention(self, i: int, qkv, positions: torch.Tensor, lengths_after: torch.Tensor, S: int, bound: int,
+                   start_bound: int) -> torch.Tensor:
+        """Layer i's projected rows (q rows of a CLA shared layer) normed, rotated
+        and appended, then attention over its (or its anchor's) cache."""
+        cfg, w, a = self.cfg, self.layers[i], self.anchor(i)
+        D, Hq, Hkv = ops.HEAD_DIM, cfg.num_heads, cfg.num_kv_heads
+        if self.shared(i):
+            q = ops.q_norm_rope(qkv, self.cos, self.sin, positions, Hq, w.q_norm, cfg.rms_norm_eps, self.order)
+        else:
+            q = ops.qk_norm_rope_append(qkv, self.cos, self.sin, positions, self.k[a], self.v[a], self.lengths,
+                                        bound, Hq, Hkv, w.q_norm, w.k_norm, cfg.rms_norm_eps, self.order)
+        if S == 1:
+            return ops.attention_decode(q.view(self.batch, Hq, D), self.k[a], self.v[a], lengths_after, bound,
+                                        self.scale, self.workspace, self.score_mode)
+        return ops.attention_prefill(q, self.k[a], self.v[a], self.lengths, start_bound, self.scale, True)
+
+    def _few_layer(self, i: int, residual: torch.Tensor, hidden: Optional[torch.Tensor], positions: torch.Tensor,
+                   lengths_after: torch.Tensor, bound: int):
+        """A decode step's layer with each add + norm inside the projection it
+        feeds: (residual after the attention half, MLP output), from the residual
+        stream and the MLP output of the layer before (None: nothing to add)."""
+        w, B, eps = self.layers[i], self.batch, self.cfg.rms_norm_eps
+        qkv, residual = ops.norm_linear(residual, hidden, w.input_norm, eps, w.qkv, w.qkv_bias)
+        attn = self._attention(i, qkv.view(B, 1, -1), positions, lengths_after, 1, bound, 0)
+        o = ops.few_linear(attn.view(B, -1), w.o)
+        act, residual = ops.norm_linear(residual, o, w.post_norm, eps, w.gate_up, gated=True)
+        return residual, ops.few_linear(act, w.down)
 
     def _run(self, x: torch.Tensor, positions: torch.Tensor, bound: int, start_bound: int,
              trace: Optional[list] = None) -> torch.Tensor:
@@ -161,15 +179,20 @@ class DecoderModel:
         x = x.contiguous().clone()       # the residual stream; the caller's tensor is not modified
         residual = x.view(B * S, H)
         lengths_after = self.lengths + S
+        few = S == 1 and self.few
         # each layer's last residual add is fused with the next layer's input
         # norm (candle's residual add then RmsNorm, as one add + norm kernel)
-        h = ops.rms_norm(residual, self.layers[0].input_norm, eps)
+        h = None if few else ops.rms_norm(residual, self.layers[0].input_norm, eps)
+        mlp = None
         for i in range(L):
-            mlp = self._layer(i, residual, h, positions, lengths_after, S, bound, start_bound)
+            if few:
+                residual, mlp = self._few_layer(i, residual, mlp, positions, lengths_after, bound)
+            else:
+                mlp = self._layer(i, residual, h, positions, lengths_after, S, bound, start_bound)
             if trace is not None:  # the layer's output is T(residual + mlp), taken by the next add
                 trace.append((residual.clone(),
                               mlp.parts.clone() if isinstance(mlp, ops.PartialProduct) else mlp.clone()))
-            if i + 1 < L:
+            if not few and i + 1 < L:
                 h = ops.add_rms_norm(residual, mlp, self.layers[i + 1].input_norm, eps)
         self.lengths.add_(S)             # every layer appended S rows per sequence
         if S == 1:                       # every row is a last position: add + final norm at once

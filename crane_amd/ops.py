@@ -705,6 +705,64 @@ def linear_silu_mul(x: torch.Tensor, gate_up: torch.Tensor) -> torch.Tensor:
     return out
 
 
+# ------------------------------------------------ one sequence's projections
+# include/crane_few.h: a decode step's projections with the add + norm in front
+# of them (and SiLU * up behind) in one launch.
+
+def few_rows_supported(rows: int, weight: torch.Tensor, norm: bool = False, gated: bool = False) -> bool:
+    """Whether norm_linear / few_linear take `rows` rows with this [N, K] weight."""
+    N, K = weight.shape
+    return weight.dtype == torch.bfloat16 and bool(_lib.lib().crane_few_supported(rows, N, K, norm, gated, _lib.BF16))
+
+
+def _few_check(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]):
+    dev = _dev(x, weight, bias)
+    if x.dim() != 2 or weight.dim() != 2 or weight.shape[1] != x.shape[1]:
+        raise CraneHipError(_lib.E_INVALID, f"x {tuple(x.shape)} does not match weight {tuple(weight.shape)}")
+    for t, name in ((x, "x"), (weight, "weight"), (bias, "bias")):
+        if t is not None:
+            _contig(t, name)
+            if t.dtype != x.dtype:
+                raise CraneHipError(_lib.E_DTYPE, f"{name} dtype {t.dtype} != {x.dtype}")
+    if bias is not None and bias.numel() != weight.shape[0]:
+        raise CraneHipError(_lib.E_INVALID, f"bias must have {weight.shape[0]} elements")
+    return dev
+
+
+def few_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """linear for x [M, K] of the shapes few_rows_supported(M, weight) takes."""
+    dev = _few_check(x, weight, bias)
+    (M, K), N = x.shape, weight.shape[0]
+    y = torch.empty((M, N), dtype=x.dtype, device=dev)
+    check(_lib.lib().crane_few_linear(x.data_ptr(), weight.data_ptr(), _ptr(bias), y.data_ptr(), M, N, K,
+                                      _dtype_code(x), _stream(dev)), "few_linear")
+    return y
+
+
+def norm_linear(residual: torch.Tensor, hidden: Optional[torch.Tensor], norm_weight: torch.Tensor, eps: float,
+                weight: torch.Tensor, bias: Optional[torch.Tensor] = None, gated: bool = False):
+    """(y, new residual): the residual add and RmsNorm (add_rms_norm; rms_norm
+    when hidden is None) and the projection (linear, or with gated
+    linear_silu_mul over a merged gate_up weight) in one launch, for the shapes
+    few_rows_supported(M, weight, True, gated) takes.  residual [M, K] is not
+    modified: the new one is another tensor (residual itself without hidden)."""
+    dev = _few_check(residual, weight, bias)
+    (M, K), N = residual.shape, weight.shape[0]
+    _dev(residual, hidden, norm_weight)
+    if norm_weight.dtype != residual.dtype or norm_weight.numel() != K or not norm_weight.is_contiguous():
+        raise CraneHipError(_lib.E_INVALID, "norm_weight must be a contiguous [K] tensor of the rows' dtype")
+    if hidden is not None and (hidden.shape != residual.shape or hidden.dtype != residual.dtype or
+                               not hidden.is_contiguous()):
+        raise CraneHipError(_lib.E_INVALID, "hidden must be contiguous and match residual")
+    out = residual if hidden is None else torch.empty_like(residual)
+    y = torch.empty((M, N // 2 if gated else N), dtype=residual.dtype, device=dev)
+    check(_lib.lib().crane_few_norm_linear(residual.data_ptr(), _ptr(hidden), norm_weight.data_ptr(),
+                                           None if hidden is None else out.data_ptr(), eps, weight.data_ptr(),
+                                           _ptr(bias), y.data_ptr(), M, N, K, gated, _dtype_code(residual),
+                                           _stream(dev)), "norm_linear")
+    return y, out
+
+
 # ---------------------------------------------------------------- sampling
 # Token selection on the logits (include/crane_sampling.h): Crane's gpu_argmax
 # (greedy) and topk_indices (top-k / top-p candidates), batched over rows.

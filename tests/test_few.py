@@ -1,0 +1,136 @@
+"""The projections of a decode step of one sequence
+(include/crane_few.h): the add + norm, the product and SiLU * up in one launch
+against the launches they stand for, and a model step that takes them against
+the same step without."""
+import numpy as np
+import pytest
+
+import cases
+from test_gemm import _case, _silu_mul_bound, _t, assert_linear_close
+
+
+def test_few_shape_query():
+    """Which shapes the one-row calls take (host logic, no GPU)."""
+    from crane_amd import _lib
+    q = _lib.lib().crane_few_supported
+    BF16, F32 = 1, 0
+    assert q(1, 4096, 1024, 1, 0, BF16) == 1      # Qwen3-0.6B qkv_proj
+    assert q(1, 24576, 4096, 1, 1, BF16) == 1     # Qwen3-8B gate_up
+    assert q(1, 4096, 12288, 0, 0, BF16) == 1     # ... and down_proj
+    assert q(1, 4096, 4608, 1, 0, BF16) == 0      # the norm's registers
+    assert q(2, 4096, 1024, 0, 0, BF16) == 0
+    assert q(0, 4096, 1024, 0, 0, BF16) == 0
+    assert q(1, 4096, 1000, 0, 0, BF16) == 0      # K not a multiple of 512
+    assert q(1, 4096, 33280, 0, 0, BF16) == 0
+    assert q(1, 4097, 1024, 1, 1, BF16) == 0      # gated: N = 2 inter
+    assert q(1, 4096, 1024, 1, 0, F32) == 0
+    L = _lib.lib()
+    assert L.crane_few_linear(16, 16, None, 16, 2, 64, 512, BF16, None) == _lib.E_INVALID
+    assert L.crane_few_linear(16, 24, None, 16, 1, 64, 512, BF16, None) == _lib.E_ALIGN
+    assert L.crane_few_linear(16, 16, None, 16, 0, 64, 512, BF16, None) == _lib.OK
+    assert L.crane_few_norm_linear(16, 32, 16, None, 1e-6, 16, None, 48, 1, 64, 512, 0, BF16, None) == _lib.E_INVALID
+    assert L.crane_few_norm_linear(16, 32, 16, 32, 1e-6, 16, None, 48, 1, 64, 512, 0, BF16, None) == _lib.E_INVALID
+    assert L.crane_few_norm_linear(16, 32, 16, 64, 1e-6, 16, 48, 48, 1, 64, 512, 1, BF16, None) == _lib.E_INVALID
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,bias", [
+    (1, 1, 512, True),        # one output: three waves have none
+    (1, 2049, 1024, False),   # two turns, the second of few waves
+    (1, 1000, 1536, True),
+    (1, 6150, 3584, True),    # four turns of 7 slices
+    (1, 515, 4096, False),    # the widest in registers
+    (1, 260, 4608, True),     # the long kernel: 9 slices, a ring of 8
+    (1, 2100, 18944, False),  # ... 37 slices over two turns
+])
+def test_few_linear(gpu, orc, M, N, K, bias):
+    from crane_amd import ops
+    print(f"few_linear M={M} N={N} K={K}", flush=True)
+    x, w, b = _case(3100 + N + K, M, N, K, "bf16", bias)
+    args = _t(x, "bf16", gpu), _t(w, "bf16", gpu), _t(b, "bf16", gpu) if bias else None
+    got = ops.few_linear(*args)
+    assert_linear_close(got.float().cpu().numpy(), x, w, b, "bf16", orc, f"few linear {M}x{N}x{K}")
+    assert bool((got == ops.few_linear(*args)).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("add", [False, True])
+@pytest.mark.parametrize("M,N,K", [(1, 2, 512), (1, 4100, 1024), (1, 3000, 2048), (1, 516, 3584), (1, 4104, 4096)])
+def test_norm_linear(gpu, orc, M, N, K, add, gated):
+    """The residual bits of add_rms_norm; the product of its normed rows.  The
+    kernel sums the squares in another order, so a row's rounded rms may be the
+    next bf16 value: then every normed element moves by at most two bf16 ulps
+    (its rounding and the product's), else none does."""
+    import torch
+    from crane_amd import ops
+    print(f"norm_linear M={M} N={N} K={K} add={add} gated={gated}", flush=True)
+    r = cases.rng(3300 + N + K)
+    x, h = (_t(cases.cast(cases.normal(r, (M, K)), "bf16"), "bf16", gpu) for _ in range(2))
+    nw = _t(cases.cast(1 + 0.1 * cases.normal(r, (K,)), "bf16"), "bf16", gpu)
+    _, w, b = _case(3400 + N + K, M, N, K, "bf16", True)
+    wd, bd = _t(w, "bf16", gpu), None if gated else _t(b, "bf16", gpu)
+    want_res = x.clone()
+    normed = ops.add_rms_norm(want_res, h, nw, 1e-6) if add else ops.rms_norm(x, nw, 1e-6)
+    x0 = x.clone()
+    y, res = ops.norm_linear(x, h if add else None, nw, 1e-6, wd, bd, gated)
+    assert torch.equal(x, x0) and torch.equal(res, want_res)
+    n = normed.float().cpu().numpy()
+    got = y.float().cpu().numpy()
+    moved = 2.0 ** -6 * (np.abs(n) @ np.abs(w).T)  # two ulps, 2^-7 each, of every term
+    if gated:
+        ref, bound = _silu_mul_bound(n, w, orc)
+        inter = N // 2
+        gu = np.abs(orc.linear(n, w, None, "bf16", fused=True))
+        slack = 1.1 * gu[:, inter:] * moved[:, :inter] + gu[:, :inter] * moved[:, inter:]
+    else:
+        ref, bound = orc.linear(n, w, b, "bf16", fused=True), (K * 2.0 ** -24) * (np.abs(n) @ np.abs(w).T) + 2.0 ** -8 * (
+            np.abs(orc.linear(n, w, b, "bf16", fused=True)) + 2.0 ** -8)
+        slack = moved
+    d = np.abs(got.astype(np.float64) - ref)
+    for m in range(M):  # a row's rms either rounds alike or not
+        assert np.all(d[m] <= bound[m]) or np.all(d[m] <= bound[m] + slack[m]), (M, N, K, m)
+    assert float(np.mean(d <= bound)) >= 1.0 / M if M > 1 else True
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("family,batch", [("qwen3", 1), ("qwen2", 1), ("hunyuan", 1)])
+def test_model_step_takes_them(gpu, family, batch):
+    """Two decode steps of a stack that takes the few-row projections against
+    the same steps of a twin without them: same cache rows written up to the
+    projections' rounding, logits within two bf16 roundings per layer."""
+    import torch
+    from crane_amd.decoder import LayerWeights
+    from crane_amd.model import DecodeGraph, DecoderModel, ModelConfig
+    hidden, Hq, Hkv, inter, L, D = 1024, 8, 2, 1536, 2, 128
+    gen = torch.Generator(device=gpu).manual_seed(5)
+    rnd = lambda *s, std=1.0: (torch.randn(s, generator=gen, device=gpu) * std).to(torch.bfloat16)
+    cla = 2 if family == "hunyuan" else 1
+    layers = []
+    for i in range(L):
+        rows = Hq * D if cla > 1 and i % cla else (Hq + 2 * Hkv) * D
+        norms = family != "qwen2"
+        layers.append(LayerWeights(1 + rnd(hidden, std=0.1), rnd(rows, hidden, std=hidden ** -0.5),
+                                   rnd(hidden, Hq * D, std=(Hq * D) ** -0.5), 1 + rnd(hidden, std=0.1),
+                                   rnd(2 * inter, hidden, std=hidden ** -0.5), rnd(hidden, inter, std=inter ** -0.5),
+                                   rnd(rows, std=0.1) if family == "qwen2" else None,
+                                   1 + rnd(D, std=0.1) if norms else None, 1 + rnd(D, std=0.1) if norms else None))
+    cfg = ModelConfig(hidden, Hq, Hkv, inter, L, family, max_position=600, cla_share_factor=cla)
+    head = rnd(512, hidden, std=hidden ** -0.5)
+    models = [DecoderModel(cfg, layers, 1 + rnd(hidden, std=0.1) * 0, head, batch, 600) for _ in range(3)]
+    assert all(m.few for m in models)
+    models[1].few = False
+    graph = DecodeGraph(models[2])
+    for step in range(2):
+        x = rnd(batch, 1, hidden)
+        pos = torch.full((batch,), step, dtype=torch.int32, device=gpu)
+        a, b = (m.step_batch_decode(x, pos) for m in models[:2])
+        graph.x.copy_(x)
+        graph.positions.copy_(pos)
+        assert torch.equal(graph.replay(), a), "replay differs from the eager step"
+        rel = float((a.float() - b.float()).norm() / b.float().norm())
+        print(f"  {family} step {step}: rel {rel:.2e}", flush=True)
+        assert rel <= 2 * L * 2.0 ** -8
+    trace = []
+    models[0].forward(x, pos, trace)
+    assert len(trace) == L and trace[0][0].shape == trace[0][1].shape == (batch, hidden)
