@@ -616,6 +616,10 @@ constexpr int kF32BN = 32;                             // keys per tile
 constexpr int kF32Row = kHeadDim * 4;                  // bytes per key row
 constexpr int kF32TileBytes = kF32BN * kF32Row;        // 16 KiB of K (or V) per tile
 constexpr int kF32Copies = kF32TileBytes / 1024 / kWaves;  // 1 KiB blocks of a tile each wave copies
+// Grids of up to this many 128-row workgroups, over more keys than two tiles,
+// take the split form: at 384 (1500 tokens of 32 heads) 276 -> 203 us, at 512 (4 x
+// 500 tokens of 32 heads) 109 -> 130; one tile (17 tokens) 9.8 -> 11.4.
+constexpr int kF32SplitBlocks = 384;
 
 // f32 tiles keep 512-byte rows of 32 16-byte chunks; chunk c of row r sits at
 // slot c ^ swz32(r), swz32 a permutation of the low 4 bits of r.  K reads (16
@@ -782,6 +786,201 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
                             oacc[db][4 * g + 3] * inv);
 }
 
+// The same walk for grids too small to fill the chip (kF32SplitBlocks): a
+// workgroup owns 32 query rows and its 4 waves split their key tiles, wave w
+// taking tiles w, w + 4, ...  A wave runs at the f32 MFMA rate by itself (128
+// MFMAs of 64 cycles a tile), so a short prompt is bound by how many SIMDs work:
+// the 128-row form gives a 731-token prompt of 16 heads 96 workgroups, the
+// longest walking all 23 tiles.  Each wave keeps a K and a V tile of its own in
+// LDS (128 KiB in all): K(next) is copied while P V runs and V(next) while the
+// scores do, each phase longer than the copy, and no barrier is needed until the
+// waves' (max, sum, O) meet at the end.  Four times the K / V reads per flop, from
+// L2.  Measured, us: 731 tokens of 16 heads 112 -> 38 (58 TFLOP/s), 2048 of 16 heads
+// 315 -> 179 (96 TFLOP/s of 157), 100 tokens after 3000 453 -> 120.
+template <bool CAUSAL, class ROWS>
+__global__ __launch_bounds__(64 * kWaves) void prefill_f32_split_kernel(
+    const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc, ROWS rows,
+    const int32_t* __restrict__ start_pos, int max_start, int S, int B, int Hq, int Hkv, float scale_log2,
+    float* __restrict__ out) {
+    static_assert(kWaves == 4, "one output block of 32 dims per wave in the merge");
+    __shared__ __attribute__((aligned(1024))) uint8_t kbuf[kWaves][kF32TileBytes];
+    __shared__ __attribute__((aligned(1024))) uint8_t vbuf[kWaves][kF32TileBytes];
+    __shared__ float2 ml[kWaves][32];
+    const int n_rep = Hq / Hkv;
+    const int n_qt = (S + 31) / 32;
+    int qt, b, hq;
+    if (!map_block(blockIdx.x, n_qt, B, Hkv, n_rep, qt, b, hq)) return;  // uniform: padding ids
+    const int kvh = hq / n_rep;
+    const int start = min(max(start_pos[b], 0), max_start);
+    const int L = start + S;
+    const int m0 = qt * 32;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = lane & 31, h = lane >> 5;
+    const int kend = CAUSAL ? min(start + m0 + 32, L) : L;  // keys any row of the tile can see
+    const int n_tiles = (kend + kF32BN - 1) / kF32BN;
+    constexpr int kTileCopies = kF32TileBytes / 1024;
+    // copy i fills rows 2 i, 2 i + 1: the lane part of the source offset, and the rows swizzle alike mod 16
+    uint32_t vofs[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int row = 2 * i + (lane >> 5);
+        vofs[i] = pinned(row * kF32Row + 16 * ((lane & 31) ^ swz32(row)));
+    }
+    const int64_t head0 = ROWS::kPaged ? 0 : rows.offset(b, Hkv, kvh, 0);
+    const __amdgpu_buffer_rsrc_t rk = make_rsrc(kc + head0, L * kF32Row);
+    const __amdgpu_buffer_rsrc_t rv = make_rsrc(vc + head0, L * kF32Row);
+    auto issue = [&](const float* pool, const __amdgpu_buffer_rsrc_t& whole, int x, uint8_t* dst)
+        __attribute__((always_inline)) {
+        __amdgpu_buffer_rsrc_t r = whole;
+        int base = x * kF32TileBytes;
+        if constexpr (ROWS::kPaged) {
+            const int key0 = x * kF32BN;
+            const int64_t off = key0 < L ? rows.offset(b, Hkv, kvh, key0) : -1;
+            r = make_rsrc(pool + (off < 0 ? 0 : off), off < 0 ? 0 : min(kF32BN, L - key0) * kF32Row);
+            base = 0;
+        }
+#pragma unroll
+        for (int i = 0; i < kTileCopies; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, dst + i * 1024, 16, vofs[i & 7], base + (i >> 3) * 16 * kF32Row,
+                                                     0, 0);
+    };
+    if (wave < n_tiles) {
+        issue(kc, rk, wave, kbuf[wave]);
+        issue(vc, rv, wave, vbuf[wave]);
+    }
+    const int qrow = m0 + n;
+    float qf[64];
+    {
+        const float* qp = q + (((int64_t)b * Hq + hq) * S + min(qrow, S - 1)) * kHeadDim + 64 * h;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const float4 v = *reinterpret_cast<const float4*>(qp + 4 * j);
+            qf[4 * j] = v.x;
+            qf[4 * j + 1] = v.y;
+            qf[4 * j + 2] = v.z;
+            qf[4 * j + 3] = v.w;
+        }
+    }
+    f32x16_v oacc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[i][r] = 0.f;
+    float m_run = -INFINITY, l_run = 0.f;
+    const int lim = CAUSAL ? min(start + qrow, L - 1) : L - 1;  // the last key this row sees
+    const int k_row = n * kF32Row;
+    const uint8_t* kb = kbuf[wave];
+    const uint8_t* vb = vbuf[wave];
+    // both halves of the wave hold keys of the same rows
+    auto other = [&](float x) __attribute__((always_inline)) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        return make_float2(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    };
+    CRANE_WAIT_VMCNT(0);  // q, and the first tiles
+    // q used here: the wait-count pass then does not wait for its loads inside
+    // the loop, where the wait would be for the tile copies in flight
+#pragma unroll
+    for (int j = 0; j < 64; ++j) asm volatile("" : "+v"(qf[j]));
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    for (int t = wave; t < n_tiles; t += kWaves) {
+        const bool more = t + kWaves < n_tiles;
+        if (t != wave) {
+            // K(t) has landed; V(t), issued after it, may fly
+            CRANE_WAIT_VMCNT(kTileCopies);
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        }
+        const int kt = t * kF32BN;
+        f32x16_v acc;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const float4 kk = *reinterpret_cast<const float4*>(kb + k_row + 16 * ((16 * h + j) ^ swz32(n)));
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.x, qf[4 * j], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.y, qf[4 * j + 1], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.z, qf[4 * j + 2], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.w, qf[4 * j + 3], acc, 0, 0, 0);
+        }
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt 0: this tile's K reads are done
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) issue(kc, rk, t + kWaves, kbuf[wave]);
+        float mx = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int key = kt + 8 * (r >> 2) + 4 * h + (r & 3);
+            acc[r] = key > lim ? -INFINITY : acc[r] * scale_log2;
+            mx = fmaxf(mx, acc[r]);
+        }
+        const float2 mo = other(mx);
+        const float m_new = fmaxf(m_run, fmaxf(mo.x, mo.y));
+        const float m_use = m_new == -INFINITY ? 0.f : m_new;  // a row with no key yet keeps p = 0
+        const float alpha = fast_exp2(m_run - m_use);
+        float rs = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            acc[r] = fast_exp2(acc[r] - m_use);
+            rs += acc[r];
+        }
+        const float2 so = other(rs);
+        l_run = l_run * alpha + (so.x + so.y);
+        m_run = m_new;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) oacc[i][r] *= alpha;
+        if (more) CRANE_WAIT_VMCNT(kTileCopies); else CRANE_WAIT_VMCNT(0);  // V(t); K(next) may fly
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int row = 8 * (r >> 2) + 4 * h + (r & 3);
+#pragma unroll
+            for (int db = 0; db < 4; ++db) {
+                const int d = 32 * db + n;
+                const float vv = *reinterpret_cast<const float*>(vb + row * kF32Row + 16 * ((d >> 2) ^ swz32(row)) +
+                                                                 4 * (d & 3));
+                oacc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv, acc[r], oacc[db], 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // this tile's V reads are done
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) issue(vc, rv, t + kWaves, vbuf[wave]);
+    }
+    // Merge: every wave leaves its O in its K tile, block db by block db, and
+    // wave w sums block w of all four in wave order.
+    float* xo = reinterpret_cast<float*>(kbuf[wave]) + lane;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) xo[64 * (16 * db + r)] = oacc[db][r];
+    if (h == 0) ml[wave][n] = make_float2(m_run, l_run);
+    __syncthreads();
+    float mm = ml[0][n].x;
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) mm = fmaxf(mm, ml[w][n].x);
+    float a[kWaves], l = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+        a[w] = ml[w][n].x == -INFINITY ? 0.f : fast_exp2(ml[w][n].x - mm);
+        l += a[w] * ml[w][n].y;
+    }
+    if (qrow >= S) return;
+    const float inv = 1.f / l;
+    float* op = out + (((int64_t)b * S + qrow) * Hq + hq) * kHeadDim + 32 * wave + 4 * h;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        float o[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            o[e] = 0.f;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w)
+                o[e] += a[w] * reinterpret_cast<const float*>(kbuf[w])[64 * (16 * wave + 4 * g + e) + lane];
+        }
+        *reinterpret_cast<float4*>(op + 8 * g) = make_float4(o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv);
+    }
+}
+
 // Compute units of the device that runs `stream` (cached per device; host
 // threads may race to fill an entry, with the same value).
 int device_cus(hipStream_t stream) {
@@ -845,14 +1044,19 @@ int attn_prefill(const void* q, const void* k_cache, const void* v_cache, const 
         const int64_t units = (int64_t)((S + kBM - 1) / kBM) * B * Hkv;
         const int64_t blocks = ((units + 7) / 8) * 8 * n_rep;
         if (blocks > 0x7fffffffLL) return CRANE_HIP_E_INVALID;
-        if (causal)
-            hipLaunchKernelGGL((prefill_f32_kernel<true, ROWS>), dim3((unsigned)blocks), dim3(64 * kWaves), 0, st,
-                               (const float*)q, (const float*)k_cache, (const float*)v_cache, rows, start_pos,
-                               (int)max_start, S, B, Hq, Hkv, sl, (float*)out);
-        else
-            hipLaunchKernelGGL((prefill_f32_kernel<false, ROWS>), dim3((unsigned)blocks), dim3(64 * kWaves), 0, st,
-                               (const float*)q, (const float*)k_cache, (const float*)v_cache, rows, start_pos,
-                               (int)max_start, S, B, Hq, Hkv, sl, (float*)out);
+#define CRANE_PREFILL_F32(kernel, n)                                                                            \
+    hipLaunchKernelGGL((kernel), dim3((unsigned)(n)), dim3(64 * kWaves), 0, st, (const float*)q,                  \
+                       (const float*)k_cache, (const float*)v_cache, rows, start_pos, (int)max_start, S, B, Hq, Hkv, \
+                       sl, (float*)out)
+        const int64_t blocks32 = ((int64_t)((S + 31) / 32) * B * Hkv + 7) / 8 * 8 * n_rep;
+        if (blocks <= kF32SplitBlocks && max_start + S > 2 * kF32BN) {
+            if (causal) CRANE_PREFILL_F32((prefill_f32_split_kernel<true, ROWS>), blocks32);
+            else CRANE_PREFILL_F32((prefill_f32_split_kernel<false, ROWS>), blocks32);
+        } else {
+            if (causal) CRANE_PREFILL_F32((prefill_f32_kernel<true, ROWS>), blocks);
+            else CRANE_PREFILL_F32((prefill_f32_kernel<false, ROWS>), blocks);
+        }
+#undef CRANE_PREFILL_F32
     }
     return launch_status(hipGetLastError());
 }

@@ -310,6 +310,39 @@ def test_prefill_parity(gpu, orc, name, B, S, Hq, Hkv, start, causal, dtype):
     assert_close(out, ref, dtype, name)
 
 
+@pytest.mark.parametrize("B,S,Hq,Hkv,start,causal", [
+    (1, 65, 2, 1, [0], True),             # three key tiles: the fourth wave has none
+    (2, 33, 4, 2, [95, 32], True),        # a second row tile of one row; tile-edge starts
+    (1, 1, 8, 8, [200], True),            # one row over 7 tiles
+    (1, 31, 4, 1, [1000], False),         # every key visible to a partial row tile
+    (3, 257, 64, 2, [0, 5, 64], True),    # 576 workgroups of 128 rows: the unsplit form
+    (25, 40, 16, 8, [0] * 25, False),     # 400 of them, non-causal
+])
+@pytest.mark.parametrize("paged", [False, True])
+def test_prefill_f32_forms(gpu, orc, B, S, Hq, Hkv, start, causal, paged):
+    """The f32 prefill with its keys split over the waves of a 32-row workgroup
+    (small grids) and with 128-row workgroups, dense and paged, at the f32 bar."""
+    import torch
+    from crane_amd import ops
+    note(f"prefill f32 forms: B={B} S={S} Hq={Hq} Hkv={Hkv} start={start} causal={causal} paged={paged}")
+    q, k, v, st = cases.prefill_case(cases.SEED0 + 350 + S, B, S, Hq, Hkv, start, dtype="f32")
+    args = i32(st, gpu), int(st.max()), cases.scale(), causal
+    if paged:
+        P, n = 256, -(-k.shape[2] // 256)
+        pad = np.full((2, B, Hkv, n * P, D), np.nan, np.float32)
+        pad[0, :, :, :k.shape[2]], pad[1, :, :, :k.shape[2]] = k, v
+        perm = np.random.default_rng(3).permutation(B * n).astype(np.int32)
+        pools = np.empty((2, B * n, Hkv, P, D), np.float32)
+        pools[:, perm] = pad.reshape(2, B, Hkv, n, P, D).transpose(0, 1, 3, 2, 4, 5).reshape(2, B * n, Hkv, P, D)
+        out = ops.attention_prefill_paged(dev_t(q, "f32", gpu), dev_t(pools[0], "f32", gpu), dev_t(pools[1], "f32", gpu),
+                                          i32(perm.reshape(B, n), gpu), *args)
+    else:
+        out = ops.attention_prefill(dev_t(q, "f32", gpu), dev_t(k, "f32", gpu), dev_t(v, "f32", gpu), *args)
+    torch.cuda.synchronize()
+    ref = orc.attn_prefill(q, k, v, st, cases.scale(), causal, "f32").reshape(B, S, Hq, D)
+    assert_close(host(out).reshape(B, S, Hq, D), ref, "f32", "f32 forms")
+
+
 LONG_ROW_KEYS = 1024  # rows that see this many keys or more: the long rows of the one-rounding switch
 
 
