@@ -2,7 +2,7 @@
 y = x W^T + b -- Crane's merged qkv_proj, whose rows feed the fused append
 (qwen3/modeling.rs:382-387; with the Qwen2.5 bias, qwen25/qwen2.rs:136-138),
 o_proj (:466, :502), the MLP projections and the lm_head; on hipBLASLt, or on
-the per-wave ring and streaming kernels for decode-shaped bf16 products.
+the per-wave ring and LDS-tile kernels for bf16 products of few rows.
 
 The oracle's linear is pinned to numpy float64 matmul (a transposed weight
 fails); the GPU is held to the oracle within the rounding bound of its two
@@ -163,10 +163,9 @@ def test_library_product_keeps_to_its_workspace(gpu, workspace):
     (3, 20480, 128, False),    # one stage
 ])
 def test_linear_streaming_parity(gpu, orc, M, N, K, bias):
-    """Wide bf16 products with few token rows run the streaming kernel
-    (M <= 32, N >= 16384, K a multiple of 128) when K is not a whole number of
-    the per-wave ring kernel's pipelines (K % 1024 != 0 here); same bar as
-    the library path."""
+    """Wide bf16 products with few token rows run the LDS-tile kernel when K
+    is not a whole number of the per-wave ring kernel's pipelines
+    (K % 1024 != 0 here); same bar as the library path."""
     from crane_amd import ops
     print(f"linear (streaming) M={M} N={N} K={K} bias={bias}", flush=True)
     x, w, b = _case(900 + M + K, M, N, K, "bf16", bias)
@@ -382,9 +381,9 @@ SEED = int(os.environ.get("CRANE_RANDOM_SEED", 0))
 def linear_draw(seed: int, i: int):
     """Draw i of the randomised decode-projection sweep: (M, N, K, bias) with
     1-32 token rows, cycling over the shapes each path takes -- the ring
-    kernel's three configurations (N <= 4096, <= 8192, wider), the streaming
-    kernel (N >= 16384, K not a multiple of 1024) and hipBLASLt (anything
-    else) -- and M N K at most 1.5e9 so the oracle finishes in seconds."""
+    kernel's three configurations (N <= 4096, <= 8192, wider), wide N with K not
+    a multiple of 1024 (the LDS-tile kernel) and anything else (that kernel or
+    hipBLASLt) -- and M N K at most 1.5e9 so the oracle finishes in seconds."""
     r = cases.rng(seed + 9100 + i)
     M = int(r.integers(1, 33))
     kind = i % 5
