@@ -98,6 +98,9 @@ SIGNATURES = {
     "crane_few_supported": ([_i64, _i64, _i64, _i, _i, _i], _i),
     "crane_few_linear": ([_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i, _vp], _i),
     "crane_few_norm_linear": ([_vp, _vp, _vp, _vp, _f, _vp, _vp, _vp, _i64, _i64, _i64, _i, _i, _vp], _i),
+    "crane_few_attn_linear_supported": ([_i64, _i, _i64, _i], _i),
+    "crane_few_attn_linear": ([_vp, _vp, _vp, _i64, _vp, _i64, _i, _i, _i, _f, _i, _vp, _sz, _vp, _vp, _vp, _i64, _i, _vp],
+                              _i),
     # include/crane_pkv.h
     "crane_pkv_create": ([_i, _i, _i, _i, _i64, _i, _i, _vpp], _i),
     "crane_pkv_destroy": ([_vp], None),

@@ -54,7 +54,8 @@
 #include <mutex>
 #include <type_traits>
 
-#include "common.h"
+#include "few_merge.h"
+#include "../../include/crane_few.h"
 
 namespace crane {
 namespace {
@@ -651,7 +652,8 @@ int launch_decode_g(const T* q, const T* kc, const T* vc, const ROWS& rows, cons
 // nsplit = ceil(max_kv / CH) chunks per sequence.
 template <typename T, int CH, class ROWS>
 int launch_decode(const T* q, const T* kc, const T* vc, const ROWS& rows, const int32_t* kv_len, int max_kv, int nsplit,
-                  int B, int Hq, int Hkv, float scale, int post, float* ws_o, float* ws_ml, T* out, hipStream_t st) {
+                  int B, int Hq, int Hkv, float scale, int post, float* ws_o, float* ws_ml, T* out, hipStream_t st,
+                  bool merge = true) {
     int rc;
     switch (pick_group(Hq / Hkv)) {
 #define CRANE_DECODE_CASE(g)                                                                                          \
@@ -670,7 +672,7 @@ int launch_decode(const T* q, const T* kc, const T* vc, const ROWS& rows, const 
 #undef CRANE_DECODE_CASE
         default: return CRANE_HIP_E_GQA;
     }
-    if (rc != CRANE_HIP_OK) return rc;
+    if (rc != CRANE_HIP_OK || !merge) return rc;
     const int n_rep = Hq / Hkv, G = pick_group(n_rep);
     const dim3 mgrid((unsigned)(Hkv * (n_rep / G)), (unsigned)B, (unsigned)G);
     if (nsplit > kMergeRegs)
@@ -822,6 +824,42 @@ extern "C" int crane_hip_attn_decode_noalloc(const void* q, const void* k_cache,
     if (rc) return rc;
     return attn_decode(q, k_cache, v_cache, DenseRows{cache_cap}, kv_len, max_kv, B, Hq, Hkv, D, scale, score_mode, ws,
                        kScratchBytes, out, dtype, stream);
+}
+
+extern "C" int crane_few_attn_linear_supported(int64_t max_kv, int Hq, int64_t N, int dtype) {
+    if (max_kv <= kChunkShort || n_splits(max_kv) > kFewMergeSplits || Hq <= 0 || Hq > kFewMergeHeads ||
+        N > kFewMergeOutputs)
+        return 0;
+    return crane_few_supported(1, N, (int64_t)Hq * kHeadDim, 0, 0, dtype);
+}
+
+extern "C" int crane_few_attn_linear(const void* q, const void* k_cache, const void* v_cache, int64_t cache_cap,
+                                     const int32_t* kv_len, int64_t max_kv, int Hq, int Hkv, int D, float scale,
+                                     int score_mode, void* workspace, size_t ws_bytes, void* attn, const void* w,
+                                     void* y, int64_t N, int dtype, void* stream) {
+    if (dtype != CRANE_HIP_F32 && dtype != CRANE_HIP_BF16) return CRANE_HIP_E_DTYPE;
+    if (D != kHeadDim) return CRANE_HIP_E_HEAD_DIM;
+    if (cache_cap <= 0 || max_kv > cache_cap) return CRANE_HIP_E_CAPACITY;
+    if (Hq <= 0 || Hkv <= 0) return CRANE_HIP_E_INVALID;
+    if (Hq % Hkv != 0) return CRANE_HIP_E_GQA;
+    if (!(scale > 0.0f) || !__builtin_isfinite(scale)) return CRANE_HIP_E_INVALID;
+    if (score_mode != CRANE_HIP_SCORE_GROUPED && score_mode != CRANE_HIP_SCORE_STANDARD) return CRANE_HIP_E_INVALID;
+    if (!crane_few_attn_linear_supported(max_kv, Hq, N, dtype)) return CRANE_HIP_E_INVALID;
+    if (!q || !k_cache || !v_cache || !kv_len || !attn || !w || !y) return CRANE_HIP_E_INVALID;
+    if (!aligned16(q) || !aligned16(k_cache) || !aligned16(v_cache) || !aligned16(attn) || !aligned16(w) ||
+        !aligned16(y))
+        return CRANE_HIP_E_ALIGN;
+    const int ns = (int)n_splits(max_kv);
+    const WsLayout l = ws_layout(1, Hq, ns, dtype);
+    if (!workspace || ws_bytes < l.total || !aligned16(workspace)) return CRANE_HIP_E_WORKSPACE;
+    float* ws_o = (float*)((char*)workspace + l.o_off);
+    float* ws_ml = (float*)((char*)workspace + l.ml_off);
+    const hipStream_t st = (hipStream_t)stream;
+    const int rc = launch_decode<bf16_t, kChunkShort>(
+        (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, DenseRows{cache_cap}, kv_len, (int)max_kv, ns,
+        1, Hq, Hkv, scale, score_mode == CRANE_HIP_SCORE_STANDARD, ws_o, ws_ml, (bf16_t*)attn, st, false);
+    if (rc) return rc;
+    return few_merge_linear({ws_o, ws_ml, kv_len, (int)max_kv, kChunkShort, ns}, attn, w, y, (int)N, Hq * kHeadDim, st);
 }
 
 extern "C" int crane_hip_attn_decode_paged(const void* q, const void* k_pool, const void* v_pool, int64_t n_pages,

@@ -22,7 +22,7 @@
 // gate_up 9.1 -> 5.1, down 4.5 -> 3.6; Qwen3-8B gate_up 37.2 -> 33.6, o 8.1 ->
 // 7.5, down (few_long_kernel) 18.2 both; Qwen2.5-7B gate_up 49 -> 42.8.  Four rows
 // do not pay (qkv 6.2 -> 8.5: the norm's arithmetic is repeated by every wave).
-#include "common.h"
+#include "few_merge.h"
 #include "../../include/crane_few.h"
 
 namespace crane {
@@ -67,6 +67,46 @@ struct FewArgs {
     int N;
 };
 
+template <int NSL, bool GATED>
+__device__ __forceinline__ void few_load(const FewArgs& p, uint4 (&wr)[NSL][GATED ? 2 : 1], int s, int row, int nout,
+                                         int lane) {
+    constexpr int K = kSlice * NSL;
+#pragma unroll
+    for (int f = 0; f < (GATED ? 2 : 1); ++f)
+        wr[s][f] = stream16(p.w + (int64_t)(row + f * nout) * K + s * kSlice + 8 * lane);
+}
+
+// The products of a wave's outputs u, u + stride, ...: wr holds the slices of u,
+// xv the row.
+template <int NSL, bool GATED>
+__device__ __forceinline__ void few_outputs(const FewArgs& p, uint4 (&wr)[NSL][GATED ? 2 : 1], const uint4 (&xv)[NSL],
+                                            int u, int stride, int nout, int lane) {
+    constexpr int F = GATED ? 2 : 1;
+    for (; u < nout; u += stride) {
+        float acc[F];
+#pragma unroll
+        for (int f = 0; f < F; ++f) acc[f] = 0.f;
+        const int next = u + stride;
+#pragma unroll
+        for (int s = 0; s < NSL; ++s) {
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                acc[f] = dot2(wr[s][f].x, xv[s].x, acc[f]);
+                acc[f] = dot2(wr[s][f].y, xv[s].y, acc[f]);
+                acc[f] = dot2(wr[s][f].z, xv[s].z, acc[f]);
+                acc[f] = dot2(wr[s][f].w, xv[s].w, acc[f]);
+            }
+            if (next < nout) few_load<NSL, GATED>(p, wr, s, next, nout, lane);
+        }
+        float v = wave_sum(acc[0]);
+        if constexpr (GATED)
+            v = silu(bf16_to_f32(f32_to_bf16(v))) * bf16_to_f32(f32_to_bf16(wave_sum(acc[F - 1])));
+        else if (p.bias)
+            v += bf16_to_f32(p.bias[u]);
+        if (lane == 0) p.y[u] = f32_to_bf16(v);
+    }
+}
+
 // One row, K = 512 NSL; wave u takes outputs u, u + waves, ...  Rounding as
 // crane_hip_add_rms_norm, crane_gemm_linear and crane_hip_silu_mul: the new
 // residual, m, x / m, the product with the norm weight, the projection (gated:
@@ -82,12 +122,8 @@ __global__ __launch_bounds__(kThreads) void few_rows_kernel(FewArgs p) {
     if (u >= nout) return;
     const bool store_residual = SRC == kFromNorm && u == 0;
     uint4 wr[NSL][F];
-    auto load = [&](int s, int row) __attribute__((always_inline)) {
 #pragma unroll
-        for (int f = 0; f < F; ++f) wr[s][f] = stream16(p.w + (int64_t)(row + f * nout) * K + s * kSlice + 8 * lane);
-    };
-#pragma unroll
-    for (int s = 0; s < NSL; ++s) load(s, u);
+    for (int s = 0; s < NSL; ++s) few_load<NSL, GATED>(p, wr, s, u, nout, lane);
     uint4 xv[NSL];
 #pragma unroll
     for (int s = 0; s < NSL; ++s) xv[s] = *reinterpret_cast<const uint4*>(p.x + s * kSlice + 8 * lane);
@@ -135,29 +171,7 @@ __global__ __launch_bounds__(kThreads) void few_rows_kernel(FewArgs p) {
             xv[s] = pack8(v);
         }
     }
-    for (; u < nout; u += stride) {
-        float acc[F];
-#pragma unroll
-        for (int f = 0; f < F; ++f) acc[f] = 0.f;
-        const int next = u + stride;
-#pragma unroll
-        for (int s = 0; s < NSL; ++s) {
-#pragma unroll
-            for (int f = 0; f < F; ++f) {
-                acc[f] = dot2(wr[s][f].x, xv[s].x, acc[f]);
-                acc[f] = dot2(wr[s][f].y, xv[s].y, acc[f]);
-                acc[f] = dot2(wr[s][f].z, xv[s].z, acc[f]);
-                acc[f] = dot2(wr[s][f].w, xv[s].w, acc[f]);
-            }
-            if (next < nout) load(s, next);
-        }
-        float v = wave_sum(acc[0]);
-        if constexpr (GATED)
-            v = silu(bf16_to_f32(f32_to_bf16(v))) * bf16_to_f32(f32_to_bf16(wave_sum(acc[F - 1])));
-        else if (p.bias)
-            v += bf16_to_f32(p.bias[u]);
-        if (lane == 0) p.y[u] = f32_to_bf16(v);
-    }
+    few_outputs<NSL, GATED>(p, wr, xv, u, stride, nout, lane);
 }
 
 // One row, K past the registers (up to 32768): x in LDS, the weight slices
@@ -205,6 +219,73 @@ __global__ __launch_bounds__(kThreads) void few_long_kernel(FewArgs p, int K) {
     }
 }
 
+// o_proj of one sequence over its split-KV attention partials: the log-sum-exp
+// merge (decode.hip's kernel 2, the same weights and roundings) runs in front
+// of the product, its row in LDS: one launch less.  Each workgroup merges the
+// whole row, the 16-byte pieces of up to 8 splits from L2, while its weights are
+// in flight.  A sequence of one chunk has its row in p.x already.  Measured with
+// the chunk kernel, 16 heads and 1024 outputs, us: 1000 keys 9.31 -> 8.76, 2000
+// keys 9.25 -> 9.00, a Qwen3-0.6B step 838 -> 800.  The lines (kFewMergeSplits,
+// kFewMergeOutputs, kFewMergeHeads): 12 splits 9.47 -> 10.10; 2048 outputs, with
+// two workgroups a CU merging, 10.3 -> 9.9 at 1000 keys but 9.8 -> 10.4 at 2000;
+// 32 heads, two pieces a thread, 12.2 -> 14.1, and 4096 outputs, where later
+// turns' weights wait for the merge, 14.8 -> 17.0.
+template <int NSL>
+__global__ __launch_bounds__(kThreads) void few_merge_kernel(FewArgs p, const bf16_t* __restrict__ po,
+                                                             const float* __restrict__ pml,
+                                                             const int32_t* __restrict__ kv_len, int max_kv, int chunk,
+                                                             int nsplit) {
+    constexpr int S = kFewMergeSplits;
+    constexpr int kPieces = NSL * kSlice / 8;
+    static_assert(kPieces <= kThreads, "one piece of the row per thread");
+    __shared__ uint4 xs[kPieces];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int stride = (int)gridDim.x * kWaves, u = (int)blockIdx.x * kWaves + wave;
+    const bool live = u < p.N;  // uniform over the wave
+    uint4 wr[NSL][1];
+    if (live) {
+#pragma unroll
+        for (int s = 0; s < NSL; ++s) few_load<NSL, false>(p, wr, s, u, p.N, lane);
+    }
+    const int nc = (min(kv_len[0], max_kv) + chunk - 1) / chunk;  // chunks the sequence has, at most nsplit
+    if (const int c = (int)threadIdx.x; c < kPieces) {  // piece c: dims 8 (c % 16) .. of head c / 16
+        const int64_t row0 = (int64_t)(c >> 4) * nsplit;
+        uint4 raw[S];
+        float2 ml[S];
+#pragma unroll
+        for (int i = 0; i < S; ++i) {  // slots past the sequence's chunks hold stale values, dropped by selects
+            const int64_t row = row0 + min(i, nsplit - 1);
+            raw[i] = *reinterpret_cast<const uint4*>(po + row * kHeadDim + 8 * (c & 15));
+            ml[i] = reinterpret_cast<const float2*>(pml)[row];
+        }
+        const uint4 one = reinterpret_cast<const uint4*>(p.x)[c];
+        float M = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < S; ++i) M = fmaxf(M, i < nc ? ml[i].x : -INFINITY);
+        float den = 0.f, n[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) n[e] = 0.f;
+#pragma unroll
+        for (int i = 0; i < S; ++i) {
+            const float w = fast_exp2(ml[i].x - M) * ml[i].y;  // a normalised partial weighs w l
+            den += i < nc ? w : 0.f;
+            float v[8];
+            unpack8(raw[i], v);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) n[e] += i < nc ? w * v[e] : 0.f;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) n[e] /= den;
+        xs[c] = nc <= 1 ? one : pack8(n);
+    }
+    __syncthreads();
+    if (!live) return;
+    uint4 xv[NSL];
+#pragma unroll
+    for (int s = 0; s < NSL; ++s) xv[s] = xs[s * (kSlice / 8) + lane];
+    few_outputs<NSL, false>(p, wr, xv, u, stride, p.N, lane);
+}
+
 // Workgroups for n outputs: at most kMaxWgs, every wave the same number of turns.
 unsigned few_grid(int n) {
     const int turns = (n + kMaxWgs * kWaves - 1) / (kMaxWgs * kWaves);
@@ -226,6 +307,19 @@ int launch_few(const FewArgs& a, int K, hipStream_t st) {
     return CRANE_HIP_E_INVALID;
 }
 
+int launch_merge(const FewArgs& a, int K, const FewMerge& m, hipStream_t st) {
+    const dim3 grid(few_grid(a.N));
+#define CRANE_MERGE_CASE(n)                                                                                       \
+    if (K == n * kSlice) {                                                                                        \
+        hipLaunchKernelGGL((few_merge_kernel<n>), grid, dim3(kThreads), 0, st, a, (const bf16_t*)m.rows, m.ml,    \
+                           m.kv_len, m.max_kv, m.chunk, m.nsplit);                                                \
+        return launch_status(hipGetLastError());                                                                  \
+    }
+    CRANE_MERGE_CASE(1) CRANE_MERGE_CASE(2) CRANE_MERGE_CASE(3) CRANE_MERGE_CASE(4)
+#undef CRANE_MERGE_CASE
+    return CRANE_HIP_E_INVALID;
+}
+
 bool few_takes(int64_t M, int64_t N, int64_t K, bool norm, bool gated, int dtype) {
     if (dtype != CRANE_HIP_BF16 || M != 1 || N < 1 || N > 0x3fffffff || K < kSlice || K % kSlice) return false;
     if (gated && N % 2) return false;
@@ -242,6 +336,16 @@ int check_few(const void* x, const void* w, const void* y, int64_t M, int64_t N,
 }
 
 }  // namespace
+
+int few_merge_linear(const FewMerge& m, const void* attn, const void* w, void* y, int N, int K, hipStream_t st) {
+    FewArgs a{};
+    a.x = (const bf16_t*)attn;
+    a.w = (const bf16_t*)w;
+    a.y = (bf16_t*)y;
+    a.N = N;
+    return launch_merge(a, K, m, st);
+}
+
 }  // namespace crane
 
 using namespace crane;

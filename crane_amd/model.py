@@ -141,9 +141,10 @@ class DecoderModel:
         return proj(ops.linear_silu_mul(h2, w.gate_up), w.down)
 
     def _attention(self, i: int, qkv, positions: torch.Tensor, lengths_after: torch.Tensor, S: int, bound: int,
-                   start_bound: int) -> torch.Tensor:
+                   start_bound: int, o: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Layer i's projected rows (q rows of a CLA shared layer) normed, rotated
-        and appended, then attention over its (or its anchor's) cache."""
+        and appended, then attention over its (or its anchor's) cache; with o (one
+        sequence's decode step) o_proj of it."""
         cfg, w, a = self.cfg, self.layers[i], self.anchor(i)
         D, Hq, Hkv = ops.HEAD_DIM, cfg.num_heads, cfg.num_kv_heads
         if self.shared(i):
@@ -151,6 +152,9 @@ class DecoderModel:
         else:
             q = ops.qk_norm_rope_append(qkv, self.cos, self.sin, positions, self.k[a], self.v[a], self.lengths,
                                         bound, Hq, Hkv, w.q_norm, w.k_norm, cfg.rms_norm_eps, self.order)
+        if o is not None:
+            return ops.attention_decode_linear(q.view(self.batch, Hq, D), self.k[a], self.v[a], lengths_after, bound, o,
+                                               self.scale, self.workspace, self.score_mode)
         if S == 1:
             return ops.attention_decode(q.view(self.batch, Hq, D), self.k[a], self.v[a], lengths_after, bound,
                                         self.scale, self.workspace, self.score_mode)
@@ -163,8 +167,7 @@ class DecoderModel:
         stream and the MLP output of the layer before (None: nothing to add)."""
         w, B, eps = self.layers[i], self.batch, self.cfg.rms_norm_eps
         qkv, residual = ops.norm_linear(residual, hidden, w.input_norm, eps, w.qkv, w.qkv_bias)
-        attn = self._attention(i, qkv.view(B, 1, -1), positions, lengths_after, 1, bound, 0)
-        o = ops.few_linear(attn.view(B, -1), w.o)
+        o = self._attention(i, qkv.view(B, 1, -1), positions, lengths_after, 1, bound, 0, w.o)
         act, residual = ops.norm_linear(residual, o, w.post_norm, eps, w.gate_up, gated=True)
         return residual, ops.few_linear(act, w.down)
 

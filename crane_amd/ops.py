@@ -767,6 +767,43 @@ def norm_linear(residual: torch.Tensor, hidden: Optional[torch.Tensor], norm_wei
     return y, out
 
 
+def attention_decode_linear(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, kv_len: torch.Tensor,
+                            max_kv: int, weight: torch.Tensor, scale: Optional[float] = None,
+                            workspace: Optional[torch.Tensor] = None,
+                            score_mode: Optional[str] = None) -> torch.Tensor:
+    """few_linear(attention_decode(q, ...), weight) [1, N] for one sequence (q
+    [1, Hq, D]); where crane_few_attn_linear_supported takes the sizes the
+    attention's partials are merged inside the product."""
+    N, Hq = weight.shape[0], q.shape[1]
+    if q.shape[0] != 1 or not _lib.lib().crane_few_attn_linear_supported(max_kv, Hq, N, _dtype_code(q)):
+        return few_linear(attention_decode(q, k_cache, v_cache, kv_len, max_kv, scale, workspace,
+                                           score_mode).view(q.shape[0], -1), weight)
+    dev = _dev(q, k_cache, v_cache, kv_len, workspace, weight)
+    if q.dim() != 3 or q.shape[2] != HEAD_DIM:
+        raise CraneHipError(_lib.E_HEAD_DIM if q.dim() == 3 else _lib.E_INVALID, "q must be [1, Hq, 128]")
+    if k_cache.shape != v_cache.shape or k_cache.dim() != 4 or k_cache.shape[0] != 1 or k_cache.shape[3] != HEAD_DIM:
+        raise CraneHipError(_lib.E_INVALID, "caches must be [1, Hkv, cap, D]")
+    if weight.dim() != 2 or weight.shape[1] != Hq * HEAD_DIM:
+        raise CraneHipError(_lib.E_INVALID, f"weight {tuple(weight.shape)} does not match {Hq} heads")
+    for t, name in ((q, "q"), (k_cache, "k_cache"), (v_cache, "v_cache"), (weight, "weight")):
+        _contig(t, name)
+        if t.dtype != q.dtype:
+            raise CraneHipError(_lib.E_DTYPE, f"{name} dtype {t.dtype} != {q.dtype}")
+    _i32(kv_len, 1, "kv_len")
+    Hkv = k_cache.shape[1]
+    scale = 1.0 / math.sqrt(HEAD_DIM) if scale is None else float(scale)
+    if workspace is None:
+        workspace = decode_workspace(dev, decode_workspace_bytes(1, Hq, Hkv, max_kv, q.dtype))
+    attn = torch.empty(Hq * HEAD_DIM, dtype=q.dtype, device=dev)
+    y = torch.empty((1, N), dtype=q.dtype, device=dev)
+    check(_lib.lib().crane_few_attn_linear(
+        q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), k_cache.shape[2], kv_len.data_ptr(), max_kv, Hq, Hkv,
+        HEAD_DIM, scale, score_mode_code(score_mode, Hq // Hkv), workspace.data_ptr(),
+        workspace.numel() * workspace.element_size(), attn.data_ptr(), weight.data_ptr(), y.data_ptr(), N,
+        _dtype_code(q), _stream(dev)), "attention_decode_linear")
+    return y
+
+
 # ---------------------------------------------------------------- sampling
 # Token selection on the logits (include/crane_sampling.h): Crane's gpu_argmax
 # (greedy) and topk_indices (top-k / top-p candidates), batched over rows.

@@ -1,7 +1,7 @@
 /*
  * crane_few.h -- C ABI of the projections of a decode step of one sequence
  * (gfx950): candle Linear (qwen3/modeling.rs:382-387, 466, 573-591),
- * optionally with the residual add and RmsNorm in front of it
+ * optionally with the residual add and RmsNorm, or decode attention, in front of it
  * (qwen3/modeling.rs:655-673) or SiLU(gate) * up behind it
  * (crane-core/src/fused_ops) in the same launch.  Results and roundings are
  * those of crane_hip_add_rms_norm (or crane_hip_rms_norm), crane_gemm_linear and
@@ -12,6 +12,7 @@
 #ifndef CRANE_FEW_H
 #define CRANE_FEW_H
 
+#include <stddef.h>
 #include <stdint.h>
 
 #ifdef __cplusplus
@@ -34,6 +35,19 @@ int crane_few_linear(const void* x, const void* w, const void* bias, void* y, in
 int crane_few_norm_linear(const void* x, const void* hidden, const void* norm_w, void* residual, float eps,
                           const void* w, const void* bias, void* y, int64_t M, int64_t N, int64_t K, int gated,
                           int dtype, void* stream);
+
+/* 1 when crane_few_attn_linear takes the sizes, else 0: bf16, 256 < max_kv <=
+ * 2048, N <= 1024, Hq a multiple of 4 up to 16. */
+int crane_few_attn_linear_supported(int64_t max_kv, int Hq, int64_t N, int dtype);
+
+/* y[1, N] = attention w[N, Hq D]^T: crane_hip_attn_decode of one sequence and
+ * crane_few_linear (o_proj), with the merge of the attention's partials inside
+ * the product.  Arguments as crane_hip_attn_decode with B = 1; attn: scratch for
+ * the attention row [Hq D] (its contents are unspecified afterwards). */
+int crane_few_attn_linear(const void* q, const void* k_cache, const void* v_cache, int64_t cache_cap,
+                          const int32_t* kv_len, int64_t max_kv, int Hq, int Hkv, int D, float scale, int score_mode,
+                          void* workspace, size_t ws_bytes, void* attn, const void* w, void* y, int64_t N, int dtype,
+                          void* stream);
 
 #ifdef __cplusplus
 }

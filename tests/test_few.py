@@ -94,6 +94,53 @@ def test_norm_linear(gpu, orc, M, N, K, add, gated):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hkv,n,max_kv,N", [
+    (4, 1, 257, 257, 1),          # two chunks, the second of one key; one output
+    (16, 8, 1000, 1064, 1024),    # 4 chunks in 5 slots
+    (16, 16, 2048, 2048, 1021),   # 8 full chunks; the last workgroup's waves partly without outputs
+    (12, 4, 1793, 2048, 1000),    # the last chunk of one key; fewer pieces than threads
+    (4, 4, 200, 2000, 61),        # one chunk: the row is the chunk kernel's
+    (8, 2, 0, 300, 96),           # an empty sequence
+])
+def test_attention_decode_linear(gpu, Hq, Hkv, n, max_kv, N):
+    """One sequence's decode attention with the merge inside o_proj against
+    the merge kernel and few_linear, over a workspace of NaN.  The merge's f32
+    sums associate differently, so a few of the row's elements may round to the
+    neighbouring bf16 value (2^-16 of them per f32 ulp; eight are allowed), and
+    y, rounded once, by one ulp more."""
+    import torch
+    from crane_amd import ops
+    print(f"attention_decode_linear Hq={Hq} Hkv={Hkv} n={n} max_kv={max_kv} N={N}", flush=True)
+    assert ops._lib.lib().crane_few_attn_linear_supported(max_kv, Hq, N, ops._lib.BF16)
+    gen = torch.Generator(device=gpu).manual_seed(41 + n)
+    rnd = lambda *s: torch.randn(s, generator=gen, device=gpu).to(torch.bfloat16)
+    q, k, v = rnd(1, Hq, 128), rnd(1, Hkv, max_kv + 8, 128), rnd(1, Hkv, max_kv + 8, 128)
+    w = rnd(N, Hq * 128)
+    length = torch.tensor([n], dtype=torch.int32, device=gpu)
+    row = ops.attention_decode(q, k, v, length, max_kv).view(1, -1)
+    want = ops.few_linear(row, w).float()
+    ws = torch.full((ops.decode_workspace_bytes(1, Hq, Hkv, max_kv) // 4 + 1,), float("nan"), device=gpu)
+    got = ops.attention_decode_linear(q, k, v, length, max_kv, w, workspace=ws).float()
+    bound = 2.0 ** -7 * want.abs() + 8 * 2.0 ** -7 * (row.float().abs() * w.float().abs()).amax(1)
+    assert bool(((got - want).abs() <= bound).all())
+
+
+def test_attention_decode_linear_query():
+    """The sizes the merging o_proj takes, and what it refuses (host logic)."""
+    from crane_amd import _lib
+    L = _lib.lib()
+    q = L.crane_few_attn_linear_supported
+    assert q(257, 16, 1024, 1) and q(2048, 4, 1, 1)
+    assert not q(256, 16, 1024, 1) and not q(2049, 16, 1024, 1) and not q(1000, 16, 1025, 1) and not q(1000, 20, 1024, 1)
+    assert not q(1000, 6, 1024, 1) and not q(1000, 16, 1024, 0) and not q(1000, 16, 0, 1)
+    call = lambda cap=1000, max_kv=1000, Hq=16, Hkv=8, D=128, ws=1 << 30, w=16, N=64, dt=1: L.crane_few_attn_linear(
+        16, 16, 16, cap, 16, max_kv, Hq, Hkv, D, 0.1, 0, 16, ws, 16, w, 16, N, dt, None)
+    assert call(cap=999) == _lib.E_CAPACITY and call(Hkv=3) == _lib.E_GQA and call(D=64) == _lib.E_HEAD_DIM
+    assert call(ws=64) == _lib.E_WORKSPACE and call(w=24) == _lib.E_ALIGN and call(dt=0) == _lib.E_INVALID
+    assert call(max_kv=200) == _lib.E_INVALID
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("family,batch", [("qwen3", 1), ("qwen2", 1), ("hunyuan", 1)])
 def test_model_step_takes_them(gpu, family, batch):
     """Two decode steps of a stack that takes the few-row projections against
