@@ -259,20 +259,23 @@ __global__ __launch_bounds__(256) void tile_gemm_kernel(TileArgs p, int tiles, i
 }
 
 template <int FT, int MT, int OUT>
-void launch_tile(const TileCfg& c, const TileArgs& a, hipStream_t st) {
+bool launch_tile(const TileCfg& c, const TileArgs& a, hipStream_t st) {
     const int nout = OUT == kTileGated ? a.N / 2 : a.N, per = OUT == kTileGated ? 16 * FT : 32 * FT;
     const int tiles = (nout + per - 1) / per, tb = (a.M + 32 * MT - 1) / (32 * MT);
     const dim3 grid((unsigned)((tiles + 7) / 8 * 8 * tb), (unsigned)c.splits);
     if (tb == 1)
         hipLaunchKernelGGL((tile_gemm_kernel<FT, MT, OUT, true>), grid, dim3(256), 0, st, a, tiles, tb);
-    else if constexpr (MT < 4)  // tile_cfg takes 4 token tiles only where they cover M
+    else if constexpr (MT < 4)
         hipLaunchKernelGGL((tile_gemm_kernel<FT, MT, OUT, false>), grid, dim3(256), 0, st, a, tiles, tb);
+    else
+        return false;  // 4 token tiles only where they cover M
+    return true;
 }
 
 template <int OUT>
 bool launch_tile_form(const TileCfg& c, const TileArgs& a, hipStream_t st) {
 #define CRANE_TILE_FORM(f, m) \
-    if (c.ft == f && c.mt == m) return launch_tile<f, m, OUT>(c, a, st), true;
+    if (c.ft == f && c.mt == m) return launch_tile<f, m, OUT>(c, a, st);
     CRANE_TILE_FORM(1, 1) CRANE_TILE_FORM(2, 1) CRANE_TILE_FORM(3, 1) CRANE_TILE_FORM(4, 1)
     CRANE_TILE_FORM(1, 2) CRANE_TILE_FORM(2, 2) CRANE_TILE_FORM(3, 2) CRANE_TILE_FORM(4, 2)
     CRANE_TILE_FORM(1, 3) CRANE_TILE_FORM(2, 3) CRANE_TILE_FORM(3, 3) CRANE_TILE_FORM(4, 3)

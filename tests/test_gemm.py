@@ -206,6 +206,29 @@ def test_linear_ring_parity(gpu, orc, M, N, K, bias):
     assert bool((got == got2).all())
 
 
+def test_tile_launch_refuses_a_form_without_a_kernel():
+    """A form that has no kernel for the row count (4 token tiles that do not
+    cover the rows, 4 feature by 4 token tiles) launches nothing and says so:
+    every product's caller returns an error instead of an unwritten output."""
+    import ctypes
+    from crane_amd import _lib
+
+    class Cfg(ctypes.Structure):
+        _fields_ = [(n, ctypes.c_int) for n in ("ft", "mt", "splits")]
+
+    class Args(ctypes.Structure):
+        _fields_ = [(n, ctypes.c_void_p) for n in ("x", "w", "bias", "y", "parts")] + \
+                   [(n, ctypes.c_int) for n in ("M", "N", "K")]
+
+    args = Args(16, 16, None, 16, 16, 129, 512, 512)
+    for out in ("rows", "gated", "parts"):
+        name = f"launch_tile_{out}"
+        launch = getattr(_lib.lib(), f"_ZN5crane{len(name)}{name}ERKNS_7TileCfgERKNS_8TileArgsEP12ihipStream_t")
+        launch.argtypes, launch.restype = [ctypes.c_void_p] * 3, ctypes.c_bool
+        for ft, mt in ((1, 4), (2, 4), (3, 4), (4, 4)):
+            assert not launch(ctypes.addressof(Cfg(ft, mt, 1)), ctypes.addressof(args), None), (out, ft, mt)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,bias", [
     (33, 4096, 64, True),      # one stage; a second token tile of one row
