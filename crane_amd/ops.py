@@ -77,11 +77,14 @@ def _i32(t: torch.Tensor, n: int, name: str) -> None:
 
 
 def _stream(dev: torch.device) -> int:
-    """The handle of the device's current stream, without the Stream object
-    (torch.cuda.current_stream(dev).cuda_stream: 1.9 us a call, twice in a decode
-    attention call whose launches take 4.5; this 0.1)."""
-    index = dev.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    """The handle of the device's current stream, for a CUDA torch.device without
+    the Stream object (torch.cuda.current_stream(dev).cuda_stream: 1.9 us a call,
+    twice in a decode attention call whose launches take 4.5; this 0.2).  Every
+    other form of a device is torch's to resolve or refuse."""
+    if type(dev) is torch.device and dev.type == "cuda":
+        index = dev.index
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    return torch.cuda.current_stream(dev).cuda_stream
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:

@@ -90,3 +90,14 @@ def test_paged_ops_reject_bad_inputs(gpu):
         p.prefill(_bf((1, Hq, 1, D), gpu))
     assert e.value.code == _lib.E_INVALID
     assert p.lengths == [0, 0]
+
+
+def test_device_forms(gpu):
+    """A workspace for a device given by name; a cache on the host is refused
+    where it needs a stream."""
+    import torch
+    from crane_amd import kv, ops
+    assert ops.decode_workspace("cuda:0", 16).device == torch.device("cuda:0")
+    ops._WORKSPACES.pop(("cuda:0", ops._stream(gpu)))
+    with pytest.raises(ValueError):
+        kv.KvCache(1, 2, device=torch.device("cpu", 0)).set_lengths([0])

@@ -50,3 +50,22 @@ def test_bad_shapes_and_cpu_step_are_rejected():
         m.forward(x, torch.zeros(1, dtype=torch.int32))
     with pytest.raises(CraneHipError):     # past the capacity
         m.forward(torch.zeros((1, 9, 256), dtype=torch.bfloat16), torch.zeros(1, dtype=torch.int32))
+
+
+def test_stream_of_any_device_form(monkeypatch):
+    """The stream lookup's short cut is for a CUDA torch.device; a string, an
+    index and a device of another type go to torch.cuda.current_stream, which
+    resolves the first two and refuses the last."""
+    from crane_amd import ops
+    asked = []
+
+    class Stream:
+        cuda_stream = 7
+
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 100 + index, raising=False)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda dev=None: asked.append(dev) or Stream)
+    assert ops._stream(torch.device("cuda:1")) == 101 and ops._stream(torch.device("cuda")) == 103
+    assert not asked
+    for dev in ("cuda:0", 0, None, torch.device("cpu"), torch.device("cpu", 0)):
+        assert ops._stream(dev) == 7 and asked.pop() is dev
