@@ -616,11 +616,6 @@ constexpr int kF32BN = 32;                             // keys per tile
 constexpr int kF32Row = kHeadDim * 4;                  // bytes per key row
 constexpr int kF32TileBytes = kF32BN * kF32Row;        // 16 KiB of K (or V) per tile
 constexpr int kF32Copies = kF32TileBytes / 1024 / kWaves;  // 1 KiB blocks of a tile each wave copies
-// Grids of up to this many 128-row workgroups, over more keys than two tiles,
-// take the split form: at 384 (1500 tokens of 32 heads) 276 -> 203 us, at 512 (4 x
-// 500 tokens of 32 heads) 109 -> 130; one tile (17 tokens) 9.8 -> 11.4.
-constexpr int kF32SplitBlocks = 384;
-
 // f32 tiles keep 512-byte rows of 32 16-byte chunks; chunk c of row r sits at
 // slot c ^ swz32(r), swz32 a permutation of the low 4 bits of r.  K reads (16
 // lanes: rows r..r+15 at one chunk index) then hit 16 different chunks, and a
@@ -786,7 +781,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
                             oacc[db][4 * g + 3] * inv);
 }
 
-// The same walk for grids too small to fill the chip (kF32SplitBlocks): a
+// The same walk for grids too small to fill the chip (prefill_f32_split): a
 // workgroup owns 32 query rows and its 4 waves split their key tiles, wave w
 // taking tiles w, w + 4, ...  A wave runs at the f32 MFMA rate by itself (128
 // MFMAs of 64 cycles a tile), so a short prompt is bound by how many SIMDs work:
@@ -981,6 +976,30 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_f32_split_kernel(
     }
 }
 
+}  // namespace
+
+// Whether an f32 call of `blocks` 128-row workgroups takes the split form.
+// Measured over 1 to 8 sequences of 17 to 2048 tokens, 4 to 32 heads, after 0 to
+// 3000 cached keys, causal and not (1052 calls):
+//   blocks <= 192:  always the faster one, 0.25 to 0.99 of the wide form's time;
+//   blocks <= 384:  causal prompts of 500 tokens or more, where it also evens out
+//                   their short and long rows (8 x 500 of 8 heads 0.81, 1500 of 32
+//                   heads 276 -> 203 us; 4 x 333 of 32 heads 69.9 -> 77.4), and up
+//                   to two row tiles, where the wide one's 128 rows are mostly
+//                   padding (8 x 33 of 32 heads after 300 keys 0.67).  Between, both
+//                   fill the chip and the wide one copies a quarter of the keys
+//                   per row: 8 x 100 of 28 heads 23.9 us against 35.1, 500 tokens
+//                   after 300, not causal, 120.7 against 145.1;
+//   past that the wide one: 512 blocks (4 x 500 of 32 heads) 109 -> 130 us.
+// Over two key tiles or fewer the split has too few tiles for its waves (17
+// tokens 9.8 -> 11.4 us).
+bool prefill_f32_split(int64_t blocks, int S, int64_t keys, bool causal) {
+    if (keys <= 2 * kF32BN) return false;
+    return blocks <= 192 || (blocks <= 384 && (S <= 64 || (causal && S >= 500)));
+}
+
+namespace {
+
 // Compute units of the device that runs `stream` (cached per device; host
 // threads may race to fill an entry, with the same value).
 int device_cus(hipStream_t stream) {
@@ -1049,7 +1068,7 @@ int attn_prefill(const void* q, const void* k_cache, const void* v_cache, const 
                        (const float*)k_cache, (const float*)v_cache, rows, start_pos, (int)max_start, S, B, Hq, Hkv, \
                        sl, (float*)out)
         const int64_t blocks32 = ((int64_t)((S + 31) / 32) * B * Hkv + 7) / 8 * 8 * n_rep;
-        if (blocks <= kF32SplitBlocks && max_start + S > 2 * kF32BN) {
+        if (prefill_f32_split(blocks, S, max_start + S, causal)) {
             if (causal) CRANE_PREFILL_F32((prefill_f32_split_kernel<true, ROWS>), blocks32);
             else CRANE_PREFILL_F32((prefill_f32_split_kernel<false, ROWS>), blocks32);
         } else {

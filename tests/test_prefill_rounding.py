@@ -344,3 +344,23 @@ def test_model_is_the_kernel_long_rows(gpu, first, causal, one_rounding):
     d = np.abs(got.astype(np.float64) - model)
     print(f"  bit-identical {same:.5f}, max |d| {d.max():.5f}", flush=True)
     assert same >= 0.99 and np.all(d <= 2.0 ** -6)
+
+
+def test_f32_form_follows_the_measured_sides():
+    """Which form an f32 prompt takes (host logic): the keys split over a 32-row
+    workgroup's waves where that measured faster than 128-row workgroups."""
+    import ctypes
+    from crane_amd import _lib
+    rule = getattr(_lib.lib(), "_ZN5crane17prefill_f32_splitElilb")
+    rule.argtypes, rule.restype = [ctypes.c_int64, ctypes.c_int, ctypes.c_int64, ctypes.c_bool], ctypes.c_bool
+
+    def split(B, Hq, Hkv, S, start, causal=True):
+        blocks = (-(-S // 128) * B * Hkv + 7) // 8 * 8 * (Hq // Hkv)
+        return rule(blocks, S, start + S, causal)
+
+    for args in [(1, 16, 8, 731, 0), (1, 16, 8, 2048, 0), (1, 32, 8, 1500, 0), (8, 8, 8, 500, 0), (1, 16, 8, 100, 3000),
+                 (8, 32, 8, 33, 300), (8, 28, 4, 17, 300, False), (1, 16, 8, 1500, 0, False)]:
+        assert split(*args), args
+    for args in [(8, 28, 4, 100, 40), (8, 32, 8, 65, 0), (4, 32, 8, 200, 300, False), (2, 28, 4, 500, 300, False),
+                 (8, 16, 8, 333, 0), (8, 16, 8, 200, 0), (1, 32, 8, 1024, 0, False), (4, 32, 8, 500, 0), (1, 16, 8, 17, 0)]:
+        assert not split(*args), args
