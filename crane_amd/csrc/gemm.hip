@@ -441,13 +441,25 @@ bool tile_takes(int64_t M, int64_t N, int64_t K, bool gated) {
     return N <= 8192 && (M <= 224 || (M <= 320 && nk <= 20000000));
 }
 
-// The form with the least time by a fit to the same sweep (2% over the best
-// form in the mean): with `per` workgroups on the busiest of 256 CUs and
-// `stages` of 64 k each, per stages (0.036 FT + 0.027 MT + 0.017 FT MT) us (its
-// copies and products) + 0.29 per, and for splits the sums' extra launch and
-// bytes.  4 token tiles only where they cover M (their second block measured
-// slower than 3), 160 features only for gate_up pairs in one round of
-// workgroups ([37888 x 3584]: 237 of them).
+}  // namespace
+
+// The form with the least of the time that the forms of a product differ in, us,
+// fitted to every form of 1324 products (1 to 320 rows, [8 .. 151936 x 64 ..
+// 28672], weights from HBM; 9% rms):
+//   per (stages (0.050 FT + 0.030 MT + 0.0046 FT MT) + 0.27 FT MT)
+//                     the copies and products of a CU, and its epilogues
+//   turns (0.023 stages + 0.69)   what waits: the ring's latency, start and end
+//   2.2 + 0.4 / MB    the splits' second launch and their f32 sums
+// with stages of 64 k and `per` workgroups on the busiest CU, of which as many as
+// LDS holds run at once (`turns` of them).  A feature tile's token blocks and
+// splits run on one XCD of 32 CUs, so `per` counts by XCD: [4608 x 3584] at 200
+// rows as 128 x 32 tiles is 252 workgroups, but 35 on four of the XCDs, and takes
+// 33.8 us where 64 x 96 tiles take 17.9.  The choice is 1.3% over the best form in
+// the geometric mean, 1.40 times at worst (counted over the whole chip 3.2% and
+// 1.88 times).  W's own read and y's store are the same for every form and left
+// out.  4 token tiles only where they cover M (their second block measured slower
+// than 3), 160 features only for gate_up pairs in one round of workgroups ([37888
+// x 3584]: 237 of them).
 TileCfg tile_cfg(int64_t M, int64_t N, int64_t K, bool gated, size_t ws_bytes) {
     TileCfg best{0, 0, 0};
     double least = 0;
@@ -458,16 +470,21 @@ TileCfg tile_cfg(int64_t M, int64_t N, int64_t K, bool gated, size_t ws_bytes) {
                 const int64_t tb = (M + 32 * mt - 1) / (32 * mt);
                 if ((tb > 1 && mt == 4) || 32 * mt >= M + 32) continue;
                 const int64_t per_tile = (gated ? 16 : 32) * ft, nout = gated ? N / 2 : N;
-                const int64_t wgs = (nout + per_tile - 1) / per_tile * tb * splits;
-                const int64_t per = (wgs + 255) / 256;
+                const int64_t tiles = (nout + per_tile - 1) / per_tile;
+                const int64_t per = ((tiles + 7) / 8 * tb * splits + 31) / 32;
                 if (ft == 5 && per > 1) continue;
-                double t = per * (K / 64.0 / splits * (0.0355 * ft + 0.0266 * mt + 0.0165 * ft * mt) + 0.29);
-                if (splits > 1) t += 2.6 + 0.65e-6 * (double)(M * N * splits * 4);
+                const int depth = 40 / (ft + mt) > 6 ? 6 : 40 / (ft + mt), resident = 40 / (depth * (ft + mt));
+                const double stages = K / 64.0 / splits;
+                double t = per * (stages * (0.050 * ft + 0.030 * mt + 0.0046 * ft * mt) + 0.27 * ft * mt) +
+                           (per + resident - 1) / resident * (0.023 * stages + 0.69);
+                if (splits > 1) t += 2.2 + 0.4e-6 * (double)(M * N * splits * 4);
                 if (!best.ft || t < least) best = TileCfg{ft, mt, splits}, least = t;
             }
     }
     return best;
 }
+
+namespace {
 
 // y = bf16(sum over splits of parts + bias), 8 features a thread: 32-bit sums
 // in split order, one rounding.  grid (ceil(N / 8 / 256), M).

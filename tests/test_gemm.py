@@ -229,6 +229,37 @@ def test_tile_launch_refuses_a_form_without_a_kernel():
             assert not launch(ctypes.addressof(Cfg(ft, mt, 1)), ctypes.addressof(args), None), (out, ft, mt)
 
 
+def tile_form(M, N, K, gated=False, ws_bytes=64 << 20):
+    """The LDS-tile kernel's form of a product of M rows and N weight rows:
+    (features / 32 per workgroup (/ 16 gated), token rows / 32, splits of K)."""
+    import ctypes
+    from crane_amd import _lib
+
+    class Cfg(ctypes.Structure):
+        _fields_ = [(n, ctypes.c_int) for n in ("ft", "mt", "splits")]
+
+    fn = getattr(_lib.lib(), "_ZN5crane8tile_cfgElllbm")
+    fn.argtypes, fn.restype = [ctypes.c_int64] * 3 + [ctypes.c_bool, ctypes.c_size_t], Cfg
+    c = fn(M, N, K, gated, ws_bytes)
+    return c.ft, c.mt, c.splits
+
+
+@pytest.mark.parametrize("M,N,K,form", [
+    (200, 4608, 3584, (2, 3, 1)),   # 17.9 us; (4, 1, 1), 252 workgroups of which 35 on each of four XCDs, 33.8
+    (257, 3584, 3584, (2, 3, 1)),   # 21.3; (4, 1, 1) 33.3
+    (320, 4096, 14336, (4, 3, 2)),  # 62.1; (2, 3, 1), 256 workgroups in 8 rounds of feature tiles, 107.9
+    (129, 2560, 9728, (3, 3, 4)),   # 23.2; (4, 2, 4) 38.6
+    (320, 1536, 8960, (3, 3, 4)),   # 22.5; (1, 2, 1) 40.3
+    (77, 4096, 12288, (2, 3, 4)),   # 27.1, the fastest by either count
+    (300, 4608, 3584, (3, 2, 1)),   # 22.6, likewise
+])
+def test_tile_form_counts_workgroups_by_xcd(M, N, K, form):
+    """Token blocks and splits of a feature tile share an XCD: the choice is a form
+    at or near the measured fastest (us in the list) also where an even spread over
+    the chip is uneven over the XCDs (host logic)."""
+    assert tile_form(M, N, K) == form
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,bias", [
     (33, 4096, 64, True),      # one stage; a second token tile of one row
