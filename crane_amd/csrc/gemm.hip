@@ -10,11 +10,11 @@
 // product is then a stream of W through the chip (2 bytes of W per 2 M flops).
 // Up to 32 rows, those whose K is a whole number of the per-wave rings
 // (K <= 8192; a Qwen3-8B decode step's qkv_proj, o_proj and gate_up) take the
-// per-wave ring kernel below; the lm_head and most others up to a few hundred
-// rows take tile_gemm.h's kernel (tile_takes has the line and both sides of
-// it); the rest hipBLASLt.  A product whose output only feeds a residual add (a
-// decode step's o_proj and down_proj) or the fused append (its qkv_proj) can
-// instead leave f32 split-K partial products for the add + norm or the append
+// per-wave ring kernel below, wide ones over a short K the streaming kernel; the
+// lm_head and most others up to a few hundred rows take tile_gemm.h's kernel
+// (tile_takes has the line and both sides of it); the rest hipBLASLt.  A product
+// whose output only feeds a residual add (a decode step's o_proj and down_proj)
+// or the fused append (its qkv_proj) can instead leave f32 split-K partial products for the add + norm or the append
 // to sum (crane_gemm_linear_split: the ring kernel's PARTIAL form).
 // Rounding: f32 accumulation, y = bf16(acc + b) (one rounding, as the
 // hipBLASLt bias epilogue).
@@ -36,12 +36,199 @@ namespace {
 constexpr size_t kDefaultWorkspace = 64u << 20;
 constexpr int kAlgoCandidates = 16;
 
-constexpr int kDecodeRows = 32;  // token rows the ring kernel takes
+constexpr int kDecodeRows = 32;  // token rows the ring and streaming kernels take
 
 __device__ __forceinline__ bf16x8_v as_bf16x8(uint4 u) { return __builtin_bit_cast(bf16x8_v, u); }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
+}
+
+// ---------------------------------------------------------------- streaming
+//
+// Wide products of few token rows over a short K (N >= 16384, K <= 1024; a small
+// model's lm_head): a workgroup's whole walk is a few stages, so what counts is
+// how soon its first bytes are asked for and how little runs after the last.
+//  - a workgroup of 4 waves owns 64 output features and all of K; wave w
+//    multiplies features 16 w .. 16 w + 15 (the A operand of
+//    v_mfma_f32_16x16x32_bf16) by the token rows (the B operand), f32
+//    accumulation: no sums cross the waves, as they do in tile_gemm.h;
+//  - K is streamed in stages of 128: the 64 W rows (256 bytes each) and the
+//    token rows of x are copied HBM -> LDS by bounds-checked buffer_load ...
+//    lds, each 1 KiB copy reading 4 whole 256-byte row pieces (x rows past M
+//    read as zero), into a ring of three stage buffers so two stages are in
+//    flight while one is multiplied;
+//  - 16-byte chunks are XOR-swizzled by row in LDS, so the 16 rows of one
+//    fragment read (ds_read_b128) fall in 16 different bank groups.
+
+constexpr int kSkStageK = 128;   // k per pipeline stage (256 bytes of every row)
+constexpr int kSkWaves = 4;      // waves per workgroup; each owns 16 output features
+constexpr int kSkRows = 16 * kSkWaves;
+
+// LDS image of one stage: rows of 256 bytes (16 chunks of 16 bytes, chunk c
+// of row r stored at slot c ^ (r & 15), so the 16 rows one fragment read
+// touches hit 16 different bank groups), W rows first, then x rows.
+template <int MT>
+struct SkStage {
+    static constexpr int kWBytes = kSkRows * 256;
+    static constexpr int kXBytes = 16 * MT * 256;
+    static constexpr int kBytes = kWBytes + kXBytes;
+    static constexpr int kCopies = kBytes / 1024 / kSkWaves;  // 1 KiB copies per wave per stage
+    static_assert(kBytes % (1024 * kSkWaves) == 0, "stage copies split evenly over the waves");
+};
+
+// The voffset of copy i of a wave: copy blk (of the stage's kBytes / 1024)
+// fills LDS bytes [1024 blk, +1024): rows 4 blk + lane / 16 of the stage, slot
+// lane % 16, from chunk slot ^ (row & 15) of that row's 256 bytes.  The stage's
+// k offset is the scalar offset; W rows read from the W resource, x rows
+// (token rows; rows past M read as zero) from the x resource.
+template <int MT>
+__device__ __forceinline__ uint32_t sk_voffset(int blk, int lane, int K) {
+    const int row = 4 * blk + (lane >> 4);
+    const int slot = lane & 15;
+    const int r = row < kSkRows ? row : row - kSkRows;
+    return (uint32_t)r * (uint32_t)K * 2u + 16u * (uint32_t)(slot ^ (r & 15));
+}
+
+// The W resource covers the workgroup's 64 rows (wb, wbytes), the x resource
+// the M token rows (xb, xbytes).
+struct SkSrc {
+    const bf16_t* wb;
+    const bf16_t* xb;
+    uint32_t wbytes, xbytes;
+};
+
+// Issue this wave's copies of one stage into `dst`; soff is the stage's byte
+// offset along k.  (Not a template: the host pass cannot form the LDS pointer
+// the copy takes.)
+__device__ __forceinline__ void sk_issue(uint8_t* dst, const SkSrc& src, const uint32_t* vofs, const bool* isw, int nc,
+                                         int wave, int soff) {
+#pragma unroll
+    for (int i = 0; i < nc; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(isw[i] ? row_rsrc(src.wb, src.wbytes) : row_rsrc(src.xb, src.xbytes),
+                                                 dst + (wave * nc + i) * 1024, 16, vofs[i], soff, 0, 0);
+}
+
+// One pipeline stage: wait for stage st (in `cur`), refill `nxt` (the buffer
+// of stage st - 1, which every wave has finished) with stage st + 2, and
+// multiply stage st.
+template <int MT>
+__device__ __forceinline__ void sk_stage(const uint8_t* cur, uint8_t* nxt, int st, int nst, const SkSrc& src,
+                                         const uint32_t (&vofs)[SkStage<MT>::kCopies],
+                                         const bool (&isw)[SkStage<MT>::kCopies], int wave, int wrow, int r, int q,
+                                         f32x4_v (&acc)[MT]) {
+    using St = SkStage<MT>;
+    // this wave's copies of stage st have landed (those of st + 1 may fly),
+    // and its LDS reads of stage st - 1 have completed (lgkmcnt 0: the
+    // compiler may have left the last products of stage st - 1, and their
+    // waits, below this point)
+    if (st + 1 < nst)
+        __builtin_amdgcn_s_waitcnt(0x0070 | (St::kCopies & 15) | ((St::kCopies >> 4) << 14));
+    else
+        __builtin_amdgcn_s_waitcnt(0x0070);
+    // Every wave's copies of stage st have landed and every wave has finished
+    // reading stage st - 1, so the refill below may overwrite it.  A plain
+    // barrier: a release fence here would wait for the copies still in flight
+    // (they count as LDS writes); the acquire fence keeps the reads below it.
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    if (st + 2 < nst) sk_issue(nxt, src, vofs, isw, St::kCopies, wave, (st + 2) * kSkStageK * 2);
+#pragma unroll
+    for (int j = 0; j < kSkStageK / 32; ++j) {
+        const int c = 4 * j + q;
+        const uint4 a = *reinterpret_cast<const uint4*>(cur + wrow * 256 + 16 * (c ^ (wrow & 15)));
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const int t = 16 * m + r;
+            const uint4 bx = *reinterpret_cast<const uint4*>(cur + St::kWBytes + t * 256 + 16 * (c ^ (t & 15)));
+            acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a), as_bf16x8(bx), acc[m], 0, 0, 0);
+        }
+    }
+}
+
+// y = x[M, K] W[N, K]^T (+ b): N / 64 workgroups of 256 threads; workgroup
+// `tile` owns features [64 tile, +64).  Wave w multiplies features 16 w .. +15
+// (the A operand) by the MT token groups of 16 (the B operand).  Lane l holds
+// A row l % 16 / B column l % 16 with the k elements of chunk (4 j + l / 16) of
+// k-step j of a stage; accumulator element i is feature 16 w + 4 (l / 16) + i
+// and token 16 m + l % 16.
+template <int MT>
+__global__ __launch_bounds__(64 * kSkWaves) void skinny_gemm_kernel(const bf16_t* __restrict__ x,
+                                                                    const bf16_t* __restrict__ w,
+                                                                    const bf16_t* __restrict__ bias,
+                                                                    bf16_t* __restrict__ y, int M, int N, int K) {
+    using St = SkStage<MT>;
+    // three stage buffers as separate objects: the compiler's wait-count pass
+    // then knows which buffer each copy writes and waits only for that one
+    __shared__ __attribute__((aligned(1024))) uint8_t lds0[St::kBytes];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds1[St::kBytes];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds2[St::kBytes];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tile = blockIdx.x;
+    const int nst = K / kSkStageK;
+    const SkSrc src{w + (int64_t)tile * kSkRows * K, x, (uint32_t)kSkRows * K * 2, (uint32_t)M * K * 2};
+    uint32_t vofs[St::kCopies];
+    bool isw[St::kCopies];
+#pragma unroll
+    for (int i = 0; i < St::kCopies; ++i) {
+        const int blk = wave * St::kCopies + i;
+        vofs[i] = sk_voffset<MT>(blk, lane, K);
+        isw[i] = 4 * blk < kSkRows;  // uniform per copy
+    }
+    const int r = lane & 15, q = lane >> 4;
+    const int wrow = 16 * wave + r;
+    f32x4_v acc[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[m] = f32x4_v{};
+    sk_issue(lds0, src, vofs, isw, St::kCopies, wave, 0);
+    if (nst > 1) sk_issue(lds1, src, vofs, isw, St::kCopies, wave, kSkStageK * 2);
+    // stage st lives in buffer st % 3; the loop is unrolled by three so every
+    // access names its buffer
+    for (int st = 0; st < nst; st += 3) {
+        sk_stage<MT>(lds0, lds2, st, nst, src, vofs, isw, wave, wrow, r, q, acc);
+        if (st + 1 < nst) sk_stage<MT>(lds1, lds0, st + 1, nst, src, vofs, isw, wave, wrow, r, q, acc);
+        if (st + 2 < nst) sk_stage<MT>(lds2, lds1, st + 2, nst, src, vofs, isw, wave, wrow, r, q, acc);
+    }
+    const int n = tile * kSkRows + 16 * wave + 4 * q;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int t = 16 * m + r;
+        if (t >= M) continue;
+        float v[4] = {acc[m][0], acc[m][1], acc[m][2], acc[m][3]};
+        if (bias) {
+            float bv[4];
+            load4(bias + n, bv);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += bv[e];
+        }
+        store4(y + (int64_t)t * N + n, v);
+    }
+}
+
+}  // namespace
+
+// Shapes: N / 64 workgroups for 256 CUs, K in whole stages, buffer offsets within
+// 32 bits.  The line in K at 13 widths of 16384 to 151936, this kernel's time
+// over tile_gemm.h's and over hipBLASLt's (geometric means of N up to 40960 and
+// past it): up to 16 rows K 256 0.78 and 0.69, 0.68 and 0.86; 640 0.92 and 0.89,
+// 0.79 and 0.97; 896 0.99 and 0.95, 0.85 and 1.01; 1152 1.03 and 1.00, 0.89 and 1.03;
+// 17 to 32 rows K 256 0.86 and 0.77, 0.79 and 0.91; 512 1.00 and 0.90, 0.93 and 1.05;
+// 640 1.02 and 0.94, 0.95 and 1.08.
+bool stream_takes(int64_t M, int64_t N, int64_t K) {
+    return M >= 1 && M <= kDecodeRows && N % kSkRows == 0 && N / kSkRows >= 256 && N <= 0x7fffffff &&
+           K % kSkStageK == 0 && K <= (M <= 16 ? 1024 : 512);
+}
+
+namespace {
+
+int launch_skinny(const bf16_t* x, const bf16_t* w, const bf16_t* bias, bf16_t* y, int M, int N, int K,
+                  hipStream_t st) {
+    const dim3 grid((unsigned)(N / kSkRows)), block(64 * kSkWaves);
+    if (M <= 16)
+        hipLaunchKernelGGL((skinny_gemm_kernel<1>), grid, block, 0, st, x, w, bias, y, M, N, K);
+    else
+        hipLaunchKernelGGL((skinny_gemm_kernel<2>), grid, block, 0, st, x, w, bias, y, M, N, K);
+    return launch_status(hipGetLastError());
 }
 
 // ---------------------------------------------------------------- per-wave rings
@@ -556,8 +743,11 @@ class Gemm {
                hipStream_t st) {
         std::lock_guard<std::mutex> lock(mu_);
         if (dtype == CRANE_HIP_BF16) {
-            const RingCfg rc = N <= kTileWideN ? ring_cfg(M, N, K) : RingCfg{0, 0, 0};
-            if (rc.ft)
+            const RingCfg rc = ring_cfg(M, N, K);
+            if (!rc.ft && stream_takes(M, N, K))
+                return launch_skinny((const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)y, (int)M, (int)N,
+                                     (int)K, st);
+            if (rc.ft && N <= kTileWideN)
                 return launch_ring<false>(rc, (const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)y,
                                           (int)M, (int)N, (int)K, st);
             if (tile_takes(M, N, K, false))

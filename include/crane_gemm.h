@@ -25,7 +25,9 @@
  *                      busiest CU the fewest features (the first listed on a
  *                      tie); gate_up + SiLU (crane_gemm_linear_silu_mul) takes
  *                      96 or 64 only
- * (the decode step's qkv_proj, o_proj, gate_up).  Else an LDS-tile kernel for N
+ * (the decode step's qkv_proj, o_proj, gate_up).  Else, up to 32 rows, a streaming
+ * kernel for N >= 16384 a multiple of 64 and K a multiple of 128 up to 1024 (M <=
+ * 16) or 512.  Else an LDS-tile kernel for N
  * a multiple of 8 and K of 64:
  *   M <= 32:   N > 8192, K > 8192 or N K <= 8 Mi;
  *   M <= 128:  every such N and K;

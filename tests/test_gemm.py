@@ -154,6 +154,27 @@ def test_library_product_keeps_to_its_workspace(gpu, workspace):
         assert bool(((y[:, n0:n0 + 9472].float() - ref).abs() <= bound).all())
 
 
+def _rule(name, nargs):
+    """One of gemm.hip's dispatch rules (host logic), by its C++ name."""
+    import ctypes
+    from crane_amd import _lib
+    fn = getattr(_lib.lib(), f"_ZN5crane{len(name)}{name}E" + "l" * nargs)
+    fn.argtypes, fn.restype = [ctypes.c_int64] * nargs, ctypes.c_bool
+    return fn
+
+
+def test_stream_rule():
+    """Wide products of few rows over a short K take the streaming kernel, at the
+    lines both of whose sides were measured."""
+    takes = _rule("stream_takes", 3)
+    for M, N, K in [(1, 151936, 896), (16, 32000, 1024), (4, 57344, 256), (32, 16384, 512), (17, 16448, 384),
+                    (1, 16384, 128)]:
+        assert takes(M, N, K), (M, N, K)
+    for M, N, K in [(1, 151936, 1152), (17, 151936, 640), (33, 32000, 256), (1, 16320, 256), (1, 32008, 256),
+                    (1, 32000, 192), (0, 32000, 256)]:
+        assert not takes(M, N, K), (M, N, K)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,bias", [
     (32, 16384, 1152, False),  # the decode batch of config 3; 9 stages of 128
@@ -163,9 +184,9 @@ def test_library_product_keeps_to_its_workspace(gpu, workspace):
     (3, 20480, 128, False),    # one stage
 ])
 def test_linear_streaming_parity(gpu, orc, M, N, K, bias):
-    """Wide bf16 products with few token rows run the LDS-tile kernel when K
-    is not a whole number of the per-wave ring kernel's pipelines
-    (K % 1024 != 0 here); same bar as the library path."""
+    """Wide bf16 products with few token rows run the streaming kernel over a
+    short K (the first of them the LDS-tile kernel) when K is not a whole number
+    of the per-wave ring kernel's pipelines; same bar as the library path."""
     from crane_amd import ops
     print(f"linear (streaming) M={M} N={N} K={K} bias={bias}", flush=True)
     x, w, b = _case(900 + M + K, M, N, K, "bf16", bias)
