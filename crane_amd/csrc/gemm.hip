@@ -508,6 +508,17 @@ RingCfg ring_cfg(int64_t M, int64_t N, int64_t K, bool gated = false) {
     return c;
 }
 
+}  // namespace
+
+// Where tile_gemm.h's kernel comes before the ring kernel: N > 32768, for more
+// than 16 token rows or K > 4096, where the x reads weigh most.  13 widths of
+// 16384 to 151936, tile against ring time (geometric mean): 17 to 32 rows 0.92
+// (K 1024) to 0.98 (2048), 0.95 (4096), 0.81 (8192); 1 to 8 rows 1.05, 1.08,
+// 1.01 and 0.85.
+bool ring_yields(int64_t M, int64_t N, int64_t K) { return N > 32768 && (M > 16 || K > 4096); }
+
+namespace {
+
 template <int MT, bool GATED>
 void launch_ring_mt(const RingCfg& c, const bf16_t* x, const bf16_t* w, const bf16_t* bias, bf16_t* y, int M, int N,
                     int K, hipStream_t st) {
@@ -747,7 +758,7 @@ class Gemm {
             if (!rc.ft && stream_takes(M, N, K))
                 return launch_skinny((const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)y, (int)M, (int)N,
                                      (int)K, st);
-            if (rc.ft && N <= kTileWideN)
+            if (rc.ft && !ring_yields(M, N, K))
                 return launch_ring<false>(rc, (const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)y,
                                           (int)M, (int)N, (int)K, st);
             if (tile_takes(M, N, K, false))

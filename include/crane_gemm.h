@@ -14,9 +14,9 @@
  * Products go to hipBLASLt with f32 accumulation, the bias added in the
  * epilogue (one rounding of acc + b, where candle rounds the product and then
  * the sum), except bf16 products with few token rows, which hand-written
- * kernels run with the same accumulation and rounding.  Up to 32 rows and
- * N = 32768: a per-wave ring kernel when K <= 8192 splits into its pipelines,
- * by these rules:
+ * kernels run with the same accumulation and rounding.  Up to 32 rows (16 where
+ * N > 32768 and K <= 4096; none where both are past): a per-wave ring kernel
+ * when K <= 8192 splits into its pipelines, by these rules:
  *   N <= 4096:         N a multiple of 16 and K of 2048;
  *   4096 < N <= 8192:  N a multiple of 32 and K of 1024;
  *   N > 8192:          of the configurations of 96 features (K a multiple of

@@ -175,6 +175,16 @@ def test_stream_rule():
         assert not takes(M, N, K), (M, N, K)
 
 
+def test_ring_rule():
+    """Wide products the ring kernel takes too go to the LDS-tile kernel only past
+    16 rows or a K of 4096."""
+    yields = _rule("ring_yields", 3)
+    for M, N, K in [(17, 151936, 2048), (32, 40960, 1024), (1, 151936, 5120), (16, 32784, 8192)]:
+        assert yields(M, N, K), (M, N, K)
+    for M, N, K in [(1, 151936, 1024), (16, 151936, 2048), (8, 40960, 4096), (32, 32768, 8192)]:
+        assert not yields(M, N, K), (M, N, K)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,bias", [
     (32, 16384, 1152, False),  # the decode batch of config 3; 9 stages of 128
