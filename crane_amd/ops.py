@@ -76,15 +76,21 @@ def _i32(t: torch.Tensor, n: int, name: str) -> None:
         raise CraneHipError(_lib.E_INVALID, f"{name} must be a contiguous int32 tensor of {n} elements")
 
 
+_CUDA_INDEX: dict = {}  # CUDA devices that carry an index (by value) -> the index
+
+
 def _stream(dev: torch.device) -> int:
     """The handle of the device's current stream, for a CUDA torch.device without
     the Stream object (torch.cuda.current_stream(dev).cuda_stream: 1.9 us a call,
-    twice in a decode attention call whose launches take 4.5; this 0.2).  Every
-    other form of a device is torch's to resolve or refuse."""
-    if type(dev) is torch.device and dev.type == "cuda":
-        index = dev.index
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
-    return torch.cuda.current_stream(dev).cuda_stream
+    twice in a decode attention call whose launches take 4.5; this 0.2, where
+    reading dev.type alone takes 0.24).  Every other form of a device is torch's to
+    resolve or refuse."""
+    index = _CUDA_INDEX.get(dev)
+    if index is None:
+        if not isinstance(dev, torch.device) or dev.type != "cuda" or dev.index is None:
+            return torch.cuda.current_stream(dev).cuda_stream
+        index = _CUDA_INDEX[dev] = dev.index
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:

@@ -63,9 +63,9 @@ def test_stream_of_any_device_form(monkeypatch):
         cuda_stream = 7
 
     monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 100 + index, raising=False)
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda dev=None: asked.append(dev) or Stream)
-    assert ops._stream(torch.device("cuda:1")) == 101 and ops._stream(torch.device("cuda")) == 103
+    for _ in range(2):
+        assert ops._stream(torch.device("cuda:1")) == 101 and ops._stream(torch.device("cuda", 0)) == 100
     assert not asked
-    for dev in ("cuda:0", 0, None, torch.device("cpu"), torch.device("cpu", 0)):
+    for dev in ("cuda:0", 0, None, torch.device("cuda"), torch.device("cpu"), torch.device("cpu", 0)):
         assert ops._stream(dev) == 7 and asked.pop() is dev
