@@ -647,37 +647,44 @@ bool tile_takes(int64_t M, int64_t N, int64_t K, bool gated) {
 //   per (stages (0.050 FT + 0.030 MT + 0.0046 FT MT) + 0.27 FT MT)
 //                     the copies and products of a CU, and its epilogues
 //   turns (0.023 stages + 0.69)   what waits: the ring's latency, start and end
-//   2.2 + 0.4 / MB    the splits' second launch and their f32 sums
+//   3.7 + 0.45 / MB   the splits' second launch and their f32 sums: 2.2 + 0.4 / MB
+//                     on the GPU by itself, the rest the host's launch, which bounds
+//                     small products called one by one (an MLP half of a 0.6B layer at
+//                     33 to 96 rows 28.5 us, 33.3 with a split down_proj), and the
+//                     weights read beside the sums
 // with stages of 64 k and `per` workgroups on the busiest CU, of which as many as
 // LDS holds run at once (`turns` of them).  A feature tile's token blocks and
 // splits run on one XCD of 32 CUs, so `per` counts by XCD: [4608 x 3584] at 200
 // rows as 128 x 32 tiles is 252 workgroups, but 35 on four of the XCDs, and takes
-// 33.8 us where 64 x 96 tiles take 17.9.  The choice is 1.3% over the best form in
-// the geometric mean, 1.40 times at worst (counted over the whole chip 3.2% and
-// 1.88 times).  W's own read and y's store are the same for every form and left
-// out.  4 token tiles only where they cover M (their second block measured slower
-// than 3), 160 features only for gate_up pairs in one round of workgroups ([37888
-// x 3584]: 237 of them).
+// 33.8 us where 64 x 96 tiles take 17.9.  On the GPU alone the choice is 1.8% over
+// the best form in the geometric mean, 1.40 times at worst (counted over the whole
+// chip 3.2% and 1.88 times).  W's own read and y's store are the same for every
+// form and left out.  4 token tiles only where they cover M (their second block
+// measured slower than 3), 160 features only for gate_up pairs in one round of
+// workgroups ([37888 x 3584]: 237 of them).
 TileCfg tile_cfg(int64_t M, int64_t N, int64_t K, bool gated, size_t ws_bytes) {
+    const uint32_t nout = (uint32_t)(gated ? N / 2 : N), rows = (uint32_t)M;
     TileCfg best{0, 0, 0};
     double least = 0;
     for (int splits = 1; splits <= (gated ? 1 : 8); splits *= 2) {
         if (K % (64 * splits) || (splits > 1 && (size_t)M * N * splits * 4 > ws_bytes)) continue;
-        for (int ft = 1; ft <= (gated ? 5 : 4); ++ft)
+        const double stages = (double)(K / 64 / splits);
+        const double sums = splits > 1 ? 3.7 + 0.45e-6 * (double)(M * N * splits * 4) : 0.0;
+        for (int ft = 1; ft <= (gated ? 5 : 4); ++ft) {
+            const uint32_t per_tile = (gated ? 16u : 32u) * (uint32_t)ft;
+            const uint32_t on_xcd = ((nout - 1) / per_tile / 8 + 1) * (uint32_t)splits;  // feature tiles x splits
             for (int mt = 1; mt <= (ft < 4 ? 4 : 3); ++mt) {
-                const int64_t tb = (M + 32 * mt - 1) / (32 * mt);
-                if ((tb > 1 && mt == 4) || 32 * mt >= M + 32) continue;
-                const int64_t per_tile = (gated ? 16 : 32) * ft, nout = gated ? N / 2 : N;
-                const int64_t tiles = (nout + per_tile - 1) / per_tile;
-                const int64_t per = ((tiles + 7) / 8 * tb * splits + 31) / 32;
+                const uint32_t tb = (rows - 1) / (32u * (uint32_t)mt) + 1;
+                if ((tb > 1 && mt == 4) || 32 * mt >= (int)rows + 32) break;
+                const uint32_t per = (on_xcd * tb + 31) / 32;
                 if (ft == 5 && per > 1) continue;
-                const int depth = 40 / (ft + mt) > 6 ? 6 : 40 / (ft + mt), resident = 40 / (depth * (ft + mt));
-                const double stages = K / 64.0 / splits;
-                double t = per * (stages * (0.050 * ft + 0.030 * mt + 0.0046 * ft * mt) + 0.27 * ft * mt) +
-                           (per + resident - 1) / resident * (0.023 * stages + 0.69);
-                if (splits > 1) t += 2.2 + 0.4e-6 * (double)(M * N * splits * 4);
+                // workgroups that LDS holds at once: rings of up to 6 stages of 4 (FT + MT) KiB
+                const uint32_t resident = ft + mt == 2 ? 3 : ft + mt == 3 ? 2 : 1;
+                const double t = per * (stages * (0.050 * ft + 0.030 * mt + 0.0046 * ft * mt) + 0.27 * ft * mt) +
+                                 ((per - 1) / resident + 1) * (0.023 * stages + 0.69) + sums;
                 if (!best.ft || t < least) best = TileCfg{ft, mt, splits}, least = t;
             }
+        }
     }
     return best;
 }

@@ -283,6 +283,7 @@ def tile_form(M, N, K, gated=False, ws_bytes=64 << 20):
     (320, 1536, 8960, (3, 3, 4)),   # 22.5; (1, 2, 1) 40.3
     (77, 4096, 12288, (2, 3, 4)),   # 27.1, the fastest by either count
     (300, 4608, 3584, (3, 2, 1)),   # 22.6, likewise
+    (77, 1024, 3072, (1, 1, 1)),    # a split saves 2 us on the GPU and costs a launch
 ])
 def test_tile_form_counts_workgroups_by_xcd(M, N, K, form):
     """Token blocks and splits of a feature tile share an XCD: the choice is a form
