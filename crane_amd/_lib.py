@@ -91,6 +91,7 @@ SIGNATURES = {
     "crane_gemm_silu_mul_supported": ([_i64, _i64, _i64, _i], _i),
     "crane_gemm_linear_silu_mul": ([_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i, _vp], _i),
     "crane_gemm_tile_silu_mul_supported": ([_i64, _i64, _i64, _i], _i),
+    "crane_gemm_tile_silu_mul_preferred": ([_i64, _i64, _i64, _i], _i),
     "crane_gemm_tile_silu_mul": ([_vp, _vp, _vp, _i64, _i64, _i64, _i, _vp], _i),
     "crane_gemm_split_supported": ([_i64, _i64, _i64, _i, _i], _i),
     "crane_gemm_linear_split": ([_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i, _i, _vp], _i),

@@ -12,10 +12,11 @@
 // (K <= 8192; a Qwen3-8B decode step's qkv_proj, o_proj and gate_up) take the
 // per-wave ring kernel below, wide ones over a short K the streaming kernel; the
 // lm_head and most others up to a few hundred rows take tile_gemm.h's kernel
-// (tile_takes has the line and both sides of it); the rest hipBLASLt.  A product
-// whose output only feeds a residual add (a decode step's o_proj and down_proj)
-// or the fused append (its qkv_proj) can instead leave f32 split-K partial products for the add + norm or the append
-// to sum (crane_gemm_linear_split: the ring kernel's PARTIAL form).
+// (tile_route has the lines and both sides of them); the rest hipBLASLt.  A
+// product whose output only feeds a residual add (a decode step's o_proj and down_proj)
+// or the fused append (its qkv_proj) can instead leave f32 split-K partial
+// products for the add + norm or the append to sum (crane_gemm_linear_split: the
+// ring kernel's PARTIAL form).
 // Rounding: f32 accumulation, y = bf16(acc + b) (one rounding, as the
 // hipBLASLt bias epilogue).
 #include <hipblaslt/hipblaslt.h>
@@ -208,15 +209,14 @@ __global__ __launch_bounds__(64 * kSkWaves) void skinny_gemm_kernel(const bf16_t
 }  // namespace
 
 // Shapes: N / 64 workgroups for 256 CUs, K in whole stages, buffer offsets within
-// 32 bits.  The line in K at 13 widths of 16384 to 151936, this kernel's time
-// over tile_gemm.h's and over hipBLASLt's (geometric means of N up to 40960 and
-// past it): up to 16 rows K 256 0.78 and 0.69, 0.68 and 0.86; 640 0.92 and 0.89,
-// 0.79 and 0.97; 896 0.99 and 0.95, 0.85 and 1.01; 1152 1.03 and 1.00, 0.89 and 1.03;
-// 17 to 32 rows K 256 0.86 and 0.77, 0.79 and 0.91; 512 1.00 and 0.90, 0.93 and 1.05;
-// 640 1.02 and 0.94, 0.95 and 1.08.
+// 32 bits.  The line in K at 13 widths of 16384 to 151936, this kernel's time over
+// tile_gemm.h's (geometric means of N up to 40960 and past it): up to 16 rows K
+// 256 0.78 and 0.69, 640 0.92 and 0.89, 896 0.99 and 0.95, 1152 1.03 and 1.00; 17
+// to 32 rows K 256 0.86 and 0.77, 640 1.01 and 0.94, 768 1.06 and 0.98.
+// (hipBLASLt is slower than both.)
 bool stream_takes(int64_t M, int64_t N, int64_t K) {
     return M >= 1 && M <= kDecodeRows && N % kSkRows == 0 && N / kSkRows >= 256 && N <= 0x7fffffff &&
-           K % kSkStageK == 0 && K <= (M <= 16 ? 1024 : 512);
+           K % kSkStageK == 0 && K <= (M <= 16 ? 1024 : 640);
 }
 
 namespace {
@@ -613,31 +613,6 @@ void launch_split(const RingCfg& c, const bf16_t* x, const bf16_t* w, float* par
 }
 
 // ---------------------------------------------------------------- tiles
-//
-// Which bf16 products take tile_gemm.h's kernel (after the ring kernel), both
-// sides measured over the Qwen3-0.6B, Qwen3-8B and Qwen2.5-7B projections at
-// 1 to 300 rows, weights read from HBM, hipBLASLt first:
-//   M <= 32:   where the library reads W slowly: gate_up pairs (63.4 -> 44.2
-//              us at [37888 x 3584]); wide N (lm_head [151936 x 4096] at 32
-//              rows 222 (ring kernel) -> 200); K > 8192 ([3584 x 18944] 105
-//              -> 27.6); small weights ([1024 x 3072] 10.1 -> 7.7).  Elsewhere
-//              ([4608 x 3584] at 20 rows: 11.6 against 12.8) the library;
-//   M <= 128:  all (1.36 times as fast in the geometric mean; the closest,
-//              [1024 x 3072] at 96 rows, 8.6 -> 8.8) but gate_up pairs wider
-//              than 32768 past 96 rows (74 -> 81);
-//   M <= 224:  N <= 8192 ([4096 x 4096] at 200 rows 21.9 -> 16.6; gate_up
-//              [24576 x 4096] at 160: 58.9 -> 65.3, so wide N stays);
-//   M <= 320:  N <= 8192 and N K <= 20 M ([4608 x 3584] at 256 rows 34.6 ->
-//              21.4, [4096 x 12288] 55.0 -> 57.5).
-constexpr int64_t kTileWideN = 32768;
-
-bool tile_takes(int64_t M, int64_t N, int64_t K, bool gated) {
-    if (M < 1 || K < 64 || K % 64 || K > (1 << 20) || N < 8 || N % (gated ? 16 : 8) || N > 0x7fffffff) return false;
-    const int64_t nk = N * K;
-    if (M <= kDecodeRows) return gated || N > 8192 || K > 8192 || nk <= (8 << 20);
-    if (M <= 128) return !gated || N <= kTileWideN || M <= 96;
-    return N <= 8192 && (M <= 224 || (M <= 320 && nk <= 20000000));
-}
 
 }  // namespace
 
@@ -662,10 +637,9 @@ bool tile_takes(int64_t M, int64_t N, int64_t K, bool gated) {
 // form and left out.  4 token tiles only where they cover M (their second block
 // measured slower than 3), 160 features only for gate_up pairs in one round of
 // workgroups ([37888 x 3584]: 237 of them).
-TileCfg tile_cfg(int64_t M, int64_t N, int64_t K, bool gated, size_t ws_bytes) {
+static TileCfg tile_best(int64_t M, int64_t N, int64_t K, bool gated, size_t ws_bytes, double& least) {
     const uint32_t nout = (uint32_t)(gated ? N / 2 : N), rows = (uint32_t)M;
     TileCfg best{0, 0, 0};
-    double least = 0;
     for (int splits = 1; splits <= (gated ? 1 : 8); splits *= 2) {
         if (K % (64 * splits) || (splits > 1 && (size_t)M * N * splits * 4 > ws_bytes)) continue;
         const double stages = (double)(K / 64 / splits);
@@ -687,6 +661,55 @@ TileCfg tile_cfg(int64_t M, int64_t N, int64_t K, bool gated, size_t ws_bytes) {
         }
     }
     return best;
+}
+
+// (the form alone)
+TileCfg tile_cfg(int64_t M, int64_t N, int64_t K, bool gated, size_t ws_bytes) {
+    double us;
+    return tile_best(M, N, K, gated, ws_bytes, us);
+}
+
+// The shapes tried: past the lines in M, N and N K the kernel was not compared over
+// the whole range, or lost at some model's shape (gate_up pairs wider than 32768
+// past 96 rows 74 -> 81 us, wide N past 128 rows 58.9 -> 65.3).
+static bool tile_takes(int64_t M, int64_t N, int64_t K, bool gated) {
+    if (M < 1 || K < 64 || K % 64 || K > (1 << 20) || N < 8 || N % (gated ? 16 : 8) || N > 0x7fffffff) return false;
+    const int64_t nk = N * K;
+    if (M <= kDecodeRows) return gated || N > 8192 || K > 8192 || nk <= (8 << 20);
+    if (M <= 128) return !gated || N <= 32768 || M <= 96;
+    return N <= 8192 && (M <= 224 || (M <= 320 && nk <= 20000000));
+}
+
+// Of those, the products the kernel takes: not where the library measured faster
+// over 8973 products of 1 to 320 rows, N 8 to 151936, K 64 to 28672, weights from
+// HBM (hipBLASLt as torch 2.10 brings it, for gate_up pairs and silu_mul).  The
+// 8672 left are 0.57 of its time in the geometric mean, 131 of them over 1.03 and 52
+// over 1.10 (1.47 at worst: its time jumps by as much between neighbouring shapes);
+// the 301 kept out 1.15.  Kept out, us, tile against library:
+//  - past 96 rows more than 24576 features, where the library's larger tiles
+//    re-read less: [57344 x 3584] at 128 rows 119, 84; gate_up [32768 x 5120] 97.6,
+//    75.7;
+//  - an output wide for its K, written late and in 8-byte pieces: [57344 x 1024]
+//    at 77 rows 33.8, 27.2; [49752 x 896] at 37 rows 23.7, 20.1;
+//  - gate_up pairs of few features over a long K, which the kernel does not split
+//    and the library does for multiples of 512: [1536 x 8192] at 1 row 17.9, 10.4;
+//    [112 x 11264] at 121 rows 25.2, 17.3; [1536 x 2048] at 4 rows 7.1, 5.9.
+// ROCm 7.2's own hipBLASLt, which a C program links, is 1.44 times as fast as
+// torch's: against that one about 1 in 10 of the products taken is over 1.10.
+TileCfg tile_route(int64_t M, int64_t N, int64_t K, bool gated, size_t ws_bytes) {
+    constexpr TileCfg no{0, 0, 0};
+    if (!tile_takes(M, N, K, gated)) return no;
+    const int64_t mb = N * K / 500000;  // of W
+    if (M > 96 && M <= 128 && N > 24576) return no;
+    if (!gated && M > kDecodeRows && M <= 128 && N > 32768 && K < 2048 &&
+        (M > 64 || (K < 1024 && N > 49152 && N <= 65536)))
+        return no;
+    const bool deep = gated && K % 512 == 0;
+    if (deep && (K >= 4096 ? M <= 16 && mb < 52 : K >= 2048 && K < 3072 && M <= 8 && mb < 13)) return no;
+    double us;
+    const TileCfg c = tile_best(M, N, K, gated, ws_bytes, us);
+    if (deep && M > kDecodeRows && K >= 5120 && us > 10 && M * N * K < 420000000) return no;
+    return c;
 }
 
 namespace {
@@ -765,12 +788,13 @@ class Gemm {
             if (!rc.ft && stream_takes(M, N, K))
                 return launch_skinny((const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)y, (int)M, (int)N,
                                      (int)K, st);
-            if (rc.ft && !ring_yields(M, N, K))
+            const TileCfg tc = rc.ft && !ring_yields(M, N, K) ? TileCfg{0, 0, 0} : tile_route(M, N, K, false, ws_bytes_);
+            if (tc.ft)
+                return linear_tile(tc, (const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)y, (int)M,
+                                   (int)N, (int)K, st);
+            if (rc.ft)
                 return launch_ring<false>(rc, (const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)y,
                                           (int)M, (int)N, (int)K, st);
-            if (tile_takes(M, N, K, false))
-                return linear_tile((const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)y, (int)M, (int)N,
-                                   (int)K, st);
         }
         Plan* p = nullptr;
         int rc = plan(M, N, K, dtype, bias != nullptr, &p);
@@ -796,9 +820,8 @@ class Gemm {
   private:
     // y = x W^T (+ b) by tile_gemm.h's kernel; with splits of K, their sums go
     // through the context's workspace.
-    int linear_tile(const bf16_t* x, const bf16_t* w, const bf16_t* bias, bf16_t* y, int M, int N, int K,
-                    hipStream_t st) {
-        const TileCfg c = tile_cfg(M, N, K, false, ws_bytes_);
+    int linear_tile(const TileCfg& c, const bf16_t* x, const bf16_t* w, const bf16_t* bias, bf16_t* y, int M, int N,
+                    int K, hipStream_t st) {
         TileArgs a{x, w, bias, y, (float*)ws_, M, N, K};
         const bool ok = c.splits == 1 ? launch_tile_rows(c, a, st) : launch_tile_parts(c, a, st);
         if (!ok) return CRANE_HIP_E_LAUNCH;
@@ -931,6 +954,11 @@ extern "C" int crane_gemm_linear_silu_mul(crane_gemm* g, const void* x, const vo
 extern "C" int crane_gemm_tile_silu_mul_supported(int64_t M, int64_t inter, int64_t K, int dtype) {
     if (dtype != CRANE_HIP_BF16 || inter <= 0 || inter > 0x3fffffffLL || inter % 8) return 0;
     return crane::tile_takes(M, 2 * inter, K, true);
+}
+
+extern "C" int crane_gemm_tile_silu_mul_preferred(int64_t M, int64_t inter, int64_t K, int dtype) {
+    return crane_gemm_tile_silu_mul_supported(M, inter, K, dtype) &&
+           crane::tile_route(M, 2 * inter, K, true, 0).ft != 0;
 }
 
 extern "C" int crane_gemm_tile_silu_mul(const void* x, const void* w, void* out, int64_t M, int64_t inter, int64_t K,

@@ -57,8 +57,10 @@ struct TileArgs {
     int M, N, K;         // N: rows of W
 };
 
-// The form a product of M rows takes (gemm.hip), splits' sums within ws_bytes.
+// The fastest form of a product of M rows (gemm.hip), the splits' sums within
+// ws_bytes; and that form where the kernel takes the product, else ft == 0.
 TileCfg tile_cfg(int64_t M, int64_t N, int64_t K, bool gated, size_t ws_bytes);
+TileCfg tile_route(int64_t M, int64_t N, int64_t K, bool gated, size_t ws_bytes);
 
 // Launch one form; false when the form is not instantiated.
 bool launch_tile_rows(const TileCfg& c, const TileArgs& a, hipStream_t st);

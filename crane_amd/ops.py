@@ -690,9 +690,9 @@ def linear_silu_mul(x: torch.Tensor, gate_up: torch.Tensor) -> torch.Tensor:
     """Crane's Mlp gate / up projections and fused_silu_mul: x [..., K] with
     the merged weight gate_up [2 I, K] (gate rows first) -> silu(gate) * up
     [..., I].  One launch where one of the library's gated kernels takes the
-    shape (decode batches and short prompts: crane_gemm_silu_mul_supported,
-    crane_gemm_tile_silu_mul_supported), else linear then silu_mul; the
-    roundings are the same either way."""
+    shape and is the faster way (decode batches and short prompts:
+    crane_gemm_silu_mul_supported, crane_gemm_tile_silu_mul_preferred), else
+    linear then silu_mul; the roundings are the same either way."""
     dev = _dev(x, gate_up)
     K = x.shape[-1]
     if gate_up.dim() != 2 or gate_up.shape[1] != K or gate_up.shape[0] % 2:
@@ -702,7 +702,7 @@ def linear_silu_mul(x: torch.Tensor, gate_up: torch.Tensor) -> torch.Tensor:
     dt = _dtype_code(x)
     lib = _lib.lib()
     ring = lib.crane_gemm_silu_mul_supported(M, inter, K, dt)
-    if not ring and not lib.crane_gemm_tile_silu_mul_supported(M, inter, K, dt):
+    if not ring and not lib.crane_gemm_tile_silu_mul_preferred(M, inter, K, dt):
         return silu_mul(linear(x, gate_up), inter)
     _contig(x, "x")
     _contig(gate_up, "gate_up")

@@ -27,18 +27,17 @@
  *                      96 or 64 only
  * (the decode step's qkv_proj, o_proj, gate_up).  Else, up to 32 rows, a streaming
  * kernel for N >= 16384 a multiple of 64 and K a multiple of 128 up to 1024 (M <=
- * 16) or 512.  Else an LDS-tile kernel for N
- * a multiple of 8 and K of 64:
+ * 16) or 640.  Else an LDS-tile kernel for N a multiple of 8 and K of 64, within
  *   M <= 32:   N > 8192, K > 8192 or N K <= 8 Mi;
  *   M <= 128:  every such N and K;
  *   M <= 224:  N <= 8192;
  *   M <= 320:  N <= 8192 and N K <= 20 M;
- * it may split K and sum the splits' f32 products through the context's
- * workspace.  The kernel that runs
- * a shape fixes the f32 summation order of its products.  A crane_gemm
- * context holds the hipBLASLt handle,
- * a workspace allocated at creation and the algorithm chosen for each shape
- * (the heuristic query runs once per shape).  Conventions otherwise as in
+ * but for products the library runs faster (gemm.hip's tile_route: N > 24576 past 96
+ * rows, wide N over a short K).  It may split K and sum the splits' f32 products
+ * through the context's workspace.  The kernel that runs a shape fixes the f32
+ * summation order of its products.  A crane_gemm context holds the hipBLASLt
+ * handle, a workspace allocated at creation and the algorithm chosen for each
+ * shape (the heuristic query runs once per shape).  Conventions otherwise as in
  * crane_hip.h; crane_gemm_linear does not allocate or synchronise.  Calls on
  * one context from several threads are serialised on the host.  Every call
  * on a context uses its one workspace, so calls whose GPU work may overlap
@@ -72,6 +71,7 @@ int crane_gemm_linear(crane_gemm* g, const void* x, const void* w, const void* b
  * multiple of 512 or inter a multiple of 32 with K a multiple of 1024 (the
  * per-wave ring kernel's gated configurations; the Qwen3-8B decode step's
  * gate_up, inter 12288, K 4096, is one).  For other shapes run
+ * crane_gemm_tile_silu_mul where crane_gemm_tile_silu_mul_preferred says so, else
  * crane_gemm_linear into a [M, 2 inter] buffer and crane_hip_silu_mul
  * (crane_layer.h). */
 int crane_gemm_silu_mul_supported(int64_t M, int64_t inter, int64_t K, int dtype);
@@ -92,6 +92,10 @@ int crane_gemm_linear_silu_mul(crane_gemm* g, const void* x, const void* w, void
  * and M <= 96 rows, or M <= 128 with inter <= 16384, or M <= 224 with
  * inter <= 4096, or M <= 320 with inter <= 4096 and 2 inter K <= 20 M. */
 int crane_gemm_tile_silu_mul_supported(int64_t M, int64_t inter, int64_t K, int dtype);
+
+/* 1 when crane_gemm_tile_silu_mul takes the shape and is expected to be faster than
+ * crane_gemm_linear and crane_hip_silu_mul, else 0. */
+int crane_gemm_tile_silu_mul_preferred(int64_t M, int64_t inter, int64_t K, int dtype);
 
 /* crane_gemm_linear_silu_mul's product, roundings and layout (its f32
  * summation order is the kernel's own); no context and no workspace. */

@@ -167,10 +167,10 @@ def test_stream_rule():
     """Wide products of few rows over a short K take the streaming kernel, at the
     lines both of whose sides were measured."""
     takes = _rule("stream_takes", 3)
-    for M, N, K in [(1, 151936, 896), (16, 32000, 1024), (4, 57344, 256), (32, 16384, 512), (17, 16448, 384),
+    for M, N, K in [(1, 151936, 896), (16, 32000, 1024), (4, 57344, 256), (32, 16384, 640), (17, 16448, 384),
                     (1, 16384, 128)]:
         assert takes(M, N, K), (M, N, K)
-    for M, N, K in [(1, 151936, 1152), (17, 151936, 640), (33, 32000, 256), (1, 16320, 256), (1, 32008, 256),
+    for M, N, K in [(1, 151936, 1152), (17, 151936, 768), (33, 32000, 256), (1, 16320, 256), (1, 32008, 256),
                     (1, 32000, 192), (0, 32000, 256)]:
         assert not takes(M, N, K), (M, N, K)
 
@@ -290,6 +290,50 @@ def test_tile_form_counts_workgroups_by_xcd(M, N, K, form):
     at or near the measured fastest (us in the list) also where an even spread over
     the chip is uneven over the XCDs (host logic)."""
     assert tile_form(M, N, K) == form
+
+
+def tile_taken(M, N, K, gated=False, ws_bytes=64 << 20):
+    """Whether a product of M rows goes to the LDS-tile kernel."""
+    import ctypes
+    from crane_amd import _lib
+
+    class Cfg(ctypes.Structure):
+        _fields_ = [(n, ctypes.c_int) for n in ("ft", "mt", "splits")]
+
+    fn = getattr(_lib.lib(), "_ZN5crane10tile_routeElllbm")
+    fn.argtypes, fn.restype = [ctypes.c_int64] * 3 + [ctypes.c_bool, ctypes.c_size_t], Cfg
+    return fn(M, N, K, gated, ws_bytes).ft != 0
+
+
+def test_tile_route_follows_the_measured_sides():
+    """Products measured slower on the LDS-tile kernel than on the library (us,
+    tile and library) stay with the library, faster ones on the kernel (host
+    logic)."""
+    from crane_amd import _lib
+    slower = [
+        (128, 57344, 3584), (128, 28672, 18944),    # 119, 84; 302, 222: wide past 96 rows
+        (77, 57344, 1024), (37, 49752, 896),        # 33.8, 27.2; 23.7, 20.1: wide over a short K
+        (321, 2048, 1024),                          # past the rows compared
+    ]
+    faster = [
+        (300, 4608, 3584), (200, 6144, 4096),       # 23.3, 23.9; 22.4, 26.3
+        (77, 24576, 4096), (77, 4096, 12288),       # 37.2, 50.0; 27.4, 42.6
+        (224, 8192, 28672), (11, 96, 18496),        # 204, 259; 35.6, 58.2
+        (128, 4096, 4096), (128, 24576, 4096),      # 16.5, 24.1; 44, 52
+        (32, 3584, 18944), (32, 151936, 4096),      # 27.6, 105; 200, 222
+        (1, 1024, 1024), (250, 1000, 768),          # small ones
+    ]
+    for shape in slower:
+        assert not tile_taken(*shape), shape
+    for shape in faster:
+        assert tile_taken(*shape), shape
+    q, s = _lib.lib().crane_gemm_tile_silu_mul_preferred, _lib.lib().crane_gemm_tile_silu_mul_supported
+    for M, inter, K in [(1, 768, 8192), (8, 1536, 4096), (121, 56, 11264)]:   # 17.9, 10.4; 11.4, 8.9; 25.2, 17.3
+        assert s(M, inter, K, 1) and not q(M, inter, K, 1), (M, inter, K)
+    assert s(128, 16384, 5120, 1) and not q(128, 16384, 5120, 1)              # 97.6, 75.7
+    for M, inter, K in [(77, 12288, 4096), (77, 3072, 1024), (20, 18944, 3584), (1, 768, 1024)]:  # 39.0, 52.7; ...
+        assert q(M, inter, K, 1), (M, inter, K)
+    assert not s(321, 1024, 1024, 1) and not q(321, 1024, 1024, 1) and not q(8, 1024, 1024, 0)
 
 
 @pytest.mark.gpu
