@@ -9,6 +9,7 @@ fails); the GPU is held to the oracle within the rounding bound of its two
 differences (f32 accumulation in another order, and one rounding of product
 + bias where candle rounds twice) and the mean-relative bar, with weights
 scaled like trained ones (std 1/sqrt(K)) so outputs are O(1)."""
+import ctypes
 import math
 import os
 
@@ -156,7 +157,6 @@ def test_library_product_keeps_to_its_workspace(gpu, workspace):
 
 def _rule(name, nargs):
     """One of gemm.hip's dispatch rules (host logic), by its C++ name."""
-    import ctypes
     from crane_amd import _lib
     fn = getattr(_lib.lib(), f"_ZN5crane{len(name)}{name}E" + "l" * nargs)
     fn.argtypes, fn.restype = [ctypes.c_int64] * nargs, ctypes.c_bool
@@ -192,6 +192,8 @@ def test_ring_rule():
     (8, 16384, 640, True),     # 5 stages: the unrolled-by-three loop's remainder of 2
     (1, 16384, 256, True),     # one token row; 2 stages
     (3, 20480, 128, False),    # one stage
+    (16, 16448, 896, True),    # 7 stages: the loop's remainder of 1; a full token group
+    (32, 16384, 640, False),   # two full token groups, the longest K for them
 ])
 def test_linear_streaming_parity(gpu, orc, M, N, K, bias):
     """Wide bf16 products with few token rows run the streaming kernel over a
@@ -218,7 +220,7 @@ def test_linear_streaming_parity(gpu, orc, M, N, K, bias):
     (32, 16384, 2048, True),   # 64 features x 4 waves (256 workgroups)
     (9, 9072, 1024, False),    # N a multiple of 48, not of 64: 48 features
     (1, 12288, 2048, False),   # one token row, wide (48 features: 256 workgroups)
-    (32, 4096, 12288, False),  # down_proj's shape: K past the ring kernel's limit, hipBLASLt
+    (32, 4096, 12288, False),  # down_proj's shape: K past the ring kernel's limit, the LDS-tile kernel in splits
 ])
 def test_linear_ring_parity(gpu, orc, M, N, K, bias):
     """bf16 products with M <= 32 token rows, N a multiple of the workgroup's
@@ -237,42 +239,47 @@ def test_linear_ring_parity(gpu, orc, M, N, K, bias):
     assert bool((got == got2).all())
 
 
+class TileCfg(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int) for n in ("ft", "mt", "splits")]
+
+
+class TileArgs(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in ("x", "w", "bias", "y", "parts")] + \
+               [(n, ctypes.c_int) for n in ("M", "N", "K")]
+
+
+def launch_tile(out, cfg, args, stream=None):
+    """One form (cfg) of the LDS-tile kernel with output "rows", "gated" or
+    "parts" (tile_gemm.h); False where it has no kernel."""
+    from crane_amd import _lib
+    name = f"launch_tile_{out}"
+    fn = getattr(_lib.lib(), f"_ZN5crane{len(name)}{name}ERKNS_7TileCfgERKNS_8TileArgsEP12ihipStream_t")
+    fn.argtypes, fn.restype = [ctypes.c_void_p] * 3, ctypes.c_bool
+    c, a = TileCfg(*cfg), TileArgs(*args)
+    return fn(ctypes.addressof(c), ctypes.addressof(a), stream)
+
+
+def _tile_rule(name, M, N, K, gated, ws_bytes):
+    from crane_amd import _lib
+    fn = getattr(_lib.lib(), f"_ZN5crane{len(name)}{name}Elllbm")
+    fn.argtypes, fn.restype = [ctypes.c_int64] * 3 + [ctypes.c_bool, ctypes.c_size_t], TileCfg
+    c = fn(M, N, K, gated, ws_bytes)
+    return c.ft, c.mt, c.splits
+
+
 def test_tile_launch_refuses_a_form_without_a_kernel():
     """A form that has no kernel for the row count (4 token tiles that do not
     cover the rows, 4 feature by 4 token tiles) launches nothing and says so:
     every product's caller returns an error instead of an unwritten output."""
-    import ctypes
-    from crane_amd import _lib
-
-    class Cfg(ctypes.Structure):
-        _fields_ = [(n, ctypes.c_int) for n in ("ft", "mt", "splits")]
-
-    class Args(ctypes.Structure):
-        _fields_ = [(n, ctypes.c_void_p) for n in ("x", "w", "bias", "y", "parts")] + \
-                   [(n, ctypes.c_int) for n in ("M", "N", "K")]
-
-    args = Args(16, 16, None, 16, 16, 129, 512, 512)
     for out in ("rows", "gated", "parts"):
-        name = f"launch_tile_{out}"
-        launch = getattr(_lib.lib(), f"_ZN5crane{len(name)}{name}ERKNS_7TileCfgERKNS_8TileArgsEP12ihipStream_t")
-        launch.argtypes, launch.restype = [ctypes.c_void_p] * 3, ctypes.c_bool
         for ft, mt in ((1, 4), (2, 4), (3, 4), (4, 4)):
-            assert not launch(ctypes.addressof(Cfg(ft, mt, 1)), ctypes.addressof(args), None), (out, ft, mt)
+            assert not launch_tile(out, (ft, mt, 1), (16, 16, None, 16, 16, 129, 512, 512)), (out, ft, mt)
 
 
 def tile_form(M, N, K, gated=False, ws_bytes=64 << 20):
     """The LDS-tile kernel's form of a product of M rows and N weight rows:
     (features / 32 per workgroup (/ 16 gated), token rows / 32, splits of K)."""
-    import ctypes
-    from crane_amd import _lib
-
-    class Cfg(ctypes.Structure):
-        _fields_ = [(n, ctypes.c_int) for n in ("ft", "mt", "splits")]
-
-    fn = getattr(_lib.lib(), "_ZN5crane8tile_cfgElllbm")
-    fn.argtypes, fn.restype = [ctypes.c_int64] * 3 + [ctypes.c_bool, ctypes.c_size_t], Cfg
-    c = fn(M, N, K, gated, ws_bytes)
-    return c.ft, c.mt, c.splits
+    return _tile_rule("tile_cfg", M, N, K, gated, ws_bytes)
 
 
 @pytest.mark.parametrize("M,N,K,form", [
@@ -294,15 +301,7 @@ def test_tile_form_counts_workgroups_by_xcd(M, N, K, form):
 
 def tile_taken(M, N, K, gated=False, ws_bytes=64 << 20):
     """Whether a product of M rows goes to the LDS-tile kernel."""
-    import ctypes
-    from crane_amd import _lib
-
-    class Cfg(ctypes.Structure):
-        _fields_ = [(n, ctypes.c_int) for n in ("ft", "mt", "splits")]
-
-    fn = getattr(_lib.lib(), "_ZN5crane10tile_routeElllbm")
-    fn.argtypes, fn.restype = [ctypes.c_int64] * 3 + [ctypes.c_bool, ctypes.c_size_t], Cfg
-    return fn(M, N, K, gated, ws_bytes).ft != 0
+    return _tile_rule("tile_route", M, N, K, gated, ws_bytes)[0] != 0
 
 
 def test_tile_route_follows_the_measured_sides():
@@ -341,9 +340,9 @@ def test_tile_route_follows_the_measured_sides():
     (33, 4096, 64, True),      # one stage; a second token tile of one row
     (40, 1000, 448, True),     # N a multiple of 8 only: a last tile of 8 features; 7 stages, ring of 6
     (64, 200, 4096, False),    # few features: 8 splits of K, two whole token tiles
-    (77, 2056, 1024, True),    # 4 splits and the bias in their sum; 13 rows of the last token tile
-    (97, 512, 2048, False),    # 4 token tiles over one block of rows
-    (129, 4096, 640, True),    # two blocks of token rows, the second of one row
+    (77, 2056, 1024, True),    # 13 rows of the last of three token tiles, each a block of its own
+    (97, 512, 2048, False),    # four blocks of one token tile, the last of one row
+    (129, 4096, 640, True),    # two blocks of 3 token tiles, the second of 33 rows
     (224, 1024, 3072, False),  # the last row count at any K
     (320, 2048, 1024, True),   # the last row count of the kernel
     (321, 2048, 1024, True),   # ... and the library's first
@@ -362,6 +361,92 @@ def test_linear_tile_parity(gpu, orc, M, N, K, bias):
     assert_linear_close(got.float().cpu().numpy(), x, w, b, "bf16", orc, f"tile linear {M}x{N}x{K}")
     got2 = ops.linear(_t(x, "bf16", gpu), _t(w, "bf16", gpu), _t(b, "bf16", gpu) if bias else None)
     assert bool((got == got2).all())
+
+
+TILE_FORMS = [(ft, mt) for ft in range(1, 5) for mt in range(1, 5 if ft < 4 else 4)]
+
+
+def _tile_shapes(ft, mt):
+    """(M, features, stages) of a form: 9 feature tiles, the last of 8 features,
+    over rows in one block and (up to 3 token tiles) two, each ending in a partial
+    tile; 2 D - 1 stages of a ring of D, a turn and the longest remainder."""
+    d = min(6, 40 // (ft + mt))
+    for M in [32 * mt - 3] + ([32 * mt + 9] if mt < 4 else []):
+        yield M, lambda per: 8 * per * ft + 8, 2 * d - 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ft,mt", TILE_FORMS)
+def test_tile_forms(gpu, orc, ft, mt):
+    """Every form of the LDS-tile kernel, launched directly: the output rows with
+    bias, and 2 splits' f32 partial products summed in split order."""
+    import torch
+    from crane_amd import ops
+    for M, features, stages in _tile_shapes(ft, mt):
+        N, K = features(32), 64 * stages
+        print(f"tile form {ft} x {mt}: M={M} N={N} K={K}", flush=True)
+        x, w, b = _case(2700 + 10 * ft + mt + M, M, N, 2 * K, "bf16", True)
+        h, wh = np.ascontiguousarray(x[:, :K]), np.ascontiguousarray(w[:, :K])
+        xd, wd, bd = _t(h, "bf16", gpu), _t(wh, "bf16", gpu), _t(b, "bf16", gpu)
+        y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=gpu)
+        assert launch_tile("rows", (ft, mt, 1), (xd.data_ptr(), wd.data_ptr(), bd.data_ptr(), y.data_ptr(), None, M, N,
+                                                 K), ops._stream(gpu))
+        assert_linear_close(y.float().cpu().numpy(), h, wh, b, "bf16", orc, f"tile rows {ft}x{mt} {M}x{N}x{K}")
+        xd, wd = _t(x, "bf16", gpu), _t(w, "bf16", gpu)
+        parts = torch.full((2, M, N), float("nan"), device=gpu)
+        assert launch_tile("parts", (ft, mt, 2), (xd.data_ptr(), wd.data_ptr(), None, None, parts.data_ptr(), M, N,
+                                                  2 * K), ops._stream(gpu))
+        got = cases.bf16((parts[0] + parts[1]).cpu().numpy())
+        assert_linear_close(got, x, w, None, "bf16", orc, f"tile parts {ft}x{mt} {M}x{N}x{2 * K}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ft,mt", TILE_FORMS + [(5, 1), (5, 2), (5, 3)])
+def test_tile_gated_forms(gpu, orc, ft, mt):
+    """Every gated form of the LDS-tile kernel, launched directly, against the
+    oracle chain within the bound of its roundings."""
+    import torch
+    from crane_amd import ops
+    for M, features, stages in _tile_shapes(ft, mt):
+        inter, K = features(16), 64 * stages
+        print(f"gated tile form {ft} x {mt}: M={M} inter={inter} K={K}", flush=True)
+        x, w, _ = _case(2900 + 10 * ft + mt + M, M, 2 * inter, K, "bf16", False)
+        xd, wd = _t(x, "bf16", gpu), _t(w, "bf16", gpu)
+        y = torch.full((M, inter), float("nan"), dtype=torch.bfloat16, device=gpu)
+        assert launch_tile("gated", (ft, mt, 1), (xd.data_ptr(), wd.data_ptr(), None, y.data_ptr(), None, M, 2 * inter,
+                                                  K), ops._stream(gpu))
+        ref, bound = _silu_mul_bound(x, w, orc)
+        got = y.float().cpu().numpy()
+        assert np.all(np.abs(got.astype(np.float64) - ref) <= bound)
+        assert float(np.mean(got == ref)) >= 0.98
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,splits,bias", [
+    (33, 200, 5760, 2, True), (12, 400, 3840, 4, True), (37, 136, 3584, 8, True), (290, 72, 3840, 4, False),
+])
+def test_linear_tile_splits(gpu, orc, M, N, K, splits, bias):
+    """Products whose K the LDS-tile kernel splits: the sums through the context's
+    workspace, with and without the bias; in a context too small for them the
+    product runs unsplit."""
+    import torch
+    from crane_amd import _lib, ops
+    assert tile_taken(M, N, K) and tile_form(M, N, K)[2] == splits and tile_form(M, N, K, ws_bytes=4096)[2] == 1
+    print(f"linear (tile, {splits} splits) M={M} N={N} K={K} bias={bias}", flush=True)
+    x, w, b = _case(3000 + M + N + K, M, N, K, "bf16", bias)
+    xd, wd, bd = _t(x, "bf16", gpu), _t(w, "bf16", gpu), _t(b, "bf16", gpu) if bias else None
+    got = ops.linear(xd, wd, bd)
+    assert_linear_close(got.float().cpu().numpy(), x, w, b, "bf16", orc, f"tile splits {M}x{N}x{K}")
+    assert torch.equal(got, ops.linear(xd, wd, bd))
+    h = ctypes.c_void_p()
+    assert _lib.lib().crane_gemm_create(4096, ctypes.byref(h)) == 0
+    try:
+        y = torch.empty_like(got)
+        assert _lib.lib().crane_gemm_linear(h, xd.data_ptr(), wd.data_ptr(), bd.data_ptr() if bias else None,
+                                            y.data_ptr(), M, N, K, _lib.BF16, ops._stream(gpu)) == 0
+        assert_linear_close(y.float().cpu().numpy(), x, w, b, "bf16", orc, f"tile unsplit {M}x{N}x{K}")
+    finally:
+        _lib.lib().crane_gemm_destroy(h)
 
 
 def test_split_shape_query():
@@ -451,8 +536,8 @@ def _silu_mul_bound(x, w, orc):
     (32, 3072, 1024),   # narrow: past the ring kernel's gated shapes
     (33, 18944, 256),   # 80 outputs a workgroup in one round
     (77, 6144, 512),    # three token tiles
-    (97, 1032, 448),    # four token tiles; 8 outputs in the last tile
-    (300, 2048, 576),   # three blocks of token rows
+    (97, 1032, 448),    # two blocks of 2 token tiles; 8 outputs in the last tile
+    (300, 2048, 576),   # four blocks of 3 token tiles
 ])
 def test_linear_silu_mul_tile_parity(gpu, orc, M, inter, K):
     """crane_gemm_tile_silu_mul against the oracle chain within the bound of
@@ -512,8 +597,8 @@ def linear_draw(seed: int, i: int):
     """Draw i of the randomised decode-projection sweep: (M, N, K, bias) with
     1-32 token rows, cycling over the shapes each path takes -- the ring
     kernel's three configurations (N <= 4096, <= 8192, wider), wide N with K not
-    a multiple of 1024 (the LDS-tile kernel) and anything else (that kernel or
-    hipBLASLt) -- and M N K at most 1.5e9 so the oracle finishes in seconds."""
+    a multiple of 1024 (the streaming and LDS-tile kernels) and anything else
+    (the latter or hipBLASLt) -- and M N K at most 1.5e9 so the oracle finishes in seconds."""
     r = cases.rng(seed + 9100 + i)
     M = int(r.integers(1, 33))
     kind = i % 5
@@ -545,6 +630,40 @@ def test_random_decode_linear(gpu, orc, i):
     assert_linear_close(got.float().cpu().numpy(), x, w, b, "bf16", orc, f"random linear {M}x{N}x{K}")
     got2 = ops.linear(_t(x, "bf16", gpu), _t(w, "bf16", gpu), _t(b, "bf16", gpu) if bias else None)
     assert bool((got == got2).all())
+
+
+def tile_draw(seed: int, i: int, gated: bool):
+    """Draw i of the LDS-tile kernel's random sweep: (M, N, K) it takes, 1 to 320
+    rows in its four row ranges, N (gated: inter) a multiple of 8 and K of 64, M N
+    K at most 8e8."""
+    r = cases.rng(seed + (9300 if gated else 9400) + i)
+    lo, hi = ((1, 32), (33, 96), (97, 128), (129, 320))[i % 4]
+    while True:
+        M = int(r.integers(lo, hi + 1))
+        N, K = 8 * int(2 ** r.uniform(0, 9.5)), 64 * int(2 ** r.uniform(0, 6.5))
+        rows = 2 * N if gated else N
+        if M * rows * K <= 8e8 and tile_taken(M, rows, K, gated, 0 if gated else 64 << 20):
+            return M, N, K
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("i", range(N_RANDOM))
+def test_random_tile_linear(gpu, orc, i):
+    """Random shapes of the LDS-tile kernel through the projections' entry points,
+    plain and gated, at the bars of the fixed shapes."""
+    from crane_amd import _lib, ops
+    M, N, K = tile_draw(SEED, i, False)
+    print(f"random tile linear {i} (seed {SEED}): M={M} N={N} K={K} {tile_form(M, N, K)}", flush=True)
+    x, w, b = _case(SEED + 9350 + i, M, N, K, "bf16", i % 2 == 0)
+    got = ops.linear(_t(x, "bf16", gpu), _t(w, "bf16", gpu), None if b is None else _t(b, "bf16", gpu))
+    assert_linear_close(got.float().cpu().numpy(), x, w, b, "bf16", orc, f"random tile linear {M}x{N}x{K}")
+    M, inter, K = tile_draw(SEED, i, True)
+    print(f"  gated: M={M} inter={inter} K={K} {tile_form(M, 2 * inter, K, True)}", flush=True)
+    assert _lib.lib().crane_gemm_tile_silu_mul_preferred(M, inter, K, 1) == 1
+    x, w, _ = _case(SEED + 9450 + i, M, 2 * inter, K, "bf16", False)
+    ref, bound = _silu_mul_bound(x, w, orc)
+    got = ops.linear_silu_mul(_t(x, "bf16", gpu), _t(w, "bf16", gpu)).float().cpu().numpy()
+    assert np.all(np.abs(got.astype(np.float64) - ref) <= bound), f"random gated tile {M}x{inter}x{K}"
 
 
 def split_draw(seed: int, i: int):
