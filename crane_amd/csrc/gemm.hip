@@ -257,10 +257,11 @@ int launch_skinny(const bf16_t* x, const bf16_t* w, const bf16_t* bias, bf16_t* 
 //                      the busiest CU the fewest tiles (gate_up: 256
 //                      workgroups of 96 features 31.8 us, 512 of 48 36.6 us,
 //                      384 of 64 42.2 us)
-// down_proj's shape [4096, 12288] stays on hipBLASLt through
-// crane_gemm_linear (26 us against 29); split over 4 ranges of K with 64
-// features per workgroup (crane_gemm_linear_split, 1 wave and a ring of 3
-// slots) it takes 18.4 us, and o_proj (2 waves, a ring of 2) 8.6 us.
+// down_proj's shape [4096, 12288] is past kRingMaxK (29 us here, 26 on
+// hipBLASLt): crane_gemm_linear runs it on LDS tiles in splits (20.8 us), and as
+// partial products over 4 ranges of K with 64 features per workgroup
+// (crane_gemm_linear_split, 1 wave and a ring of 3 slots) it takes 18.3 us; o_proj
+// (2 waves, a ring of 2) 8.7 us.
 
 constexpr int kRingMaxK = 8192;
 

@@ -2,14 +2,15 @@
 // (y = x W^T) on LDS tiles and MFMA; instantiated by tile_rows.hip,
 // tile_gated.hip and tile_parts.hip, dispatched by gemm.hip.
 //
-// What bounds it: the read of W.  Up to about 100 rows a product does under
-// 200 flops per byte of W, so the kernel is a stream of W from HBM with the
+// What bounds it: the read of W.  A product of M rows does M flops per byte of
+// W, against some 300 where the matrix cores would bound it (2.5 PFLOP/s over 8
+// TB/s): up to a few hundred rows the kernel is a stream of W from HBM, with the
 // token rows re-read from L2 by every workgroup.
 //  - A workgroup of 4 waves owns 32 FT features x 32 MT token rows.  K is
 //    walked in stages of 64 (128 bytes of every row): the W rows and the x rows
 //    of a stage go to LDS by bounds-checked buffer_load ... lds (rows past N or
 //    M read as zero), into a ring of up to 6 stages with all but one in flight
-//    (48-96 KiB per CU: what the HBM latency needs).
+//    (40 KiB a workgroup for one tile by one, 112 to 128 for the wide forms).
 //  - The waves split the stage's 64 k between them, 16 each: one
 //    v_mfma_f32_32x32x16_bf16 per (feature tile, token tile) and stage, and
 //    every byte of a stage is read from LDS exactly once.  The four k slices

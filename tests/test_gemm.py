@@ -2,7 +2,7 @@
 y = x W^T + b -- Crane's merged qkv_proj, whose rows feed the fused append
 (qwen3/modeling.rs:382-387; with the Qwen2.5 bias, qwen25/qwen2.rs:136-138),
 o_proj (:466, :502), the MLP projections and the lm_head; on hipBLASLt, or on
-the per-wave ring and LDS-tile kernels for bf16 products of few rows.
+the per-wave ring, streaming and LDS-tile kernels for bf16 products of few rows.
 
 The oracle's linear is pinned to numpy float64 matmul (a transposed weight
 fails); the GPU is held to the oracle within the rounding bound of its two
@@ -227,7 +227,7 @@ def test_linear_ring_parity(gpu, orc, M, N, K, bias):
     16/32 or 48/64/96 features (N <= 4096 / <= 8192 / wider) and K <= 8192 a
     whole number of the per-wave rings (K % 2048 == 0 for the narrowest, 1024
     or 512 for the others) run the per-wave ring kernel: the decode step's qkv_proj,
-    o_proj, gate_up and lm_head.  Same bar as the library path, and a second
+    o_proj and gate_up (a longer K takes the LDS tiles).  Same bar as the library path, and a second
     call repeats the bits (the waves' partial products are added in a fixed
     order)."""
     from crane_amd import ops
