@@ -304,8 +304,8 @@ def bench_gemm(args, dev, stream, lib):
     """The projections (include/crane_gemm.h): Qwen2.5-7B qkv_proj (with bias)
     and o_proj at config 4's 8 x 4096 rows (hipBLASLt), and at config 3's 32
     decode rows the Qwen3-8B qkv_proj, o_proj, gate_up (alone, and with the
-    SiLU*mul in the same launch) and lm_head (the per-wave ring kernel) and
-    down_proj (hipBLASLt).  The decode shapes rotate
+    SiLU*mul in the same launch; the per-wave ring kernel), lm_head and
+    down_proj (the LDS-tile kernel).  The decode shapes rotate
     over enough weight copies (> 600 MB) that every launch streams its weight
     from HBM, not from the 256 MB Infinity Cache."""
     import ctypes
