@@ -618,12 +618,15 @@ void launch_split(const RingCfg& c, const bf16_t* x, const bf16_t* w, float* par
 }  // namespace
 
 // The form with the least of the time that the forms of a product differ in, us,
-// fitted to every form of 1324 products (1 to 320 rows, [8 .. 151936 x 64 ..
-// 28672], weights from HBM; 9% rms):
-//   per (stages (0.050 FT + 0.030 MT + 0.0046 FT MT) + 0.27 FT MT)
-//                     the copies and products of a CU, and its epilogues
-//   turns (0.023 stages + 0.69)   what waits: the ring's latency, start and end
-//   3.7 + 0.45 / MB   the splits' second launch and their f32 sums: 2.2 + 0.4 / MB
+// fitted to every form of 1841 products (1 to 320 rows, [8 .. 151936 x 64 ..
+// 28672], weights from HBM):
+//   per (stages (0.058 FT + 0.039 MT + 0.0175 FT MT) + 0.32 FT MT)
+//                     the copies and products of a CU, and its epilogues; the token
+//                     rows cost 0.0095 MT more a stage where they come in several
+//                     blocks ([3584 x 18944] at 200 rows: 128 x 64 tiles 63.4 us, 96 x
+//                     96 tiles, as many workgroups, 72.8)
+//   turns (0.010 stages + 0.95)   what waits: the ring's latency, start and end
+//   4.6 + 0.45 / MB   the splits' second launch and their f32 sums: 2.2 + 0.4 / MB
 //                     on the GPU by itself, the rest the host's launch, which bounds
 //                     small products called one by one (an MLP half of a 0.6B layer at
 //                     33 to 96 rows 28.5 us, 33.3 with a split down_proj), and the
@@ -634,7 +637,9 @@ void launch_split(const RingCfg& c, const bf16_t* x, const bf16_t* w, float* par
 // rows as 128 x 32 tiles is 252 workgroups, but 35 on four of the XCDs, and takes
 // 33.8 us where 64 x 96 tiles take 17.9.  On the GPU alone the choice is 1.8% over
 // the best form in the geometric mean, 1.40 times at worst (counted over the whole
-// chip 3.2% and 1.88 times).  W's own read and y's store are the same for every
+// chip 3.2% and 1.88 times; 8 of the 1841 were over 1.03 times as fast that way,
+// 1.08 at most).  K is split only in forms whose whole tiles leave CUs idle
+// ([37888 x 12288] at 32 rows: 161.7 us, in 4 splits 180.1).  W's own read and y's store are the same for every
 // form and left out.  4 token tiles only where they cover M (their second block
 // measured slower than 3), 160 features only for gate_up pairs in one round of
 // workgroups ([37888 x 3584]: 237 of them).
@@ -644,19 +649,21 @@ static TileCfg tile_best(int64_t M, int64_t N, int64_t K, bool gated, size_t ws_
     for (int splits = 1; splits <= (gated ? 1 : 8); splits *= 2) {
         if (K % (64 * splits) || (splits > 1 && (size_t)M * N * splits * 4 > ws_bytes)) continue;
         const double stages = (double)(K / 64 / splits);
-        const double sums = splits > 1 ? 3.7 + 0.45e-6 * (double)(M * N * splits * 4) : 0.0;
+        const double sums = splits > 1 ? 4.6 + 0.45e-6 * (double)(M * N * splits * 4) : 0.0;
         for (int ft = 1; ft <= (gated ? 5 : 4); ++ft) {
             const uint32_t per_tile = (gated ? 16u : 32u) * (uint32_t)ft;
-            const uint32_t on_xcd = ((nout - 1) / per_tile / 8 + 1) * (uint32_t)splits;  // feature tiles x splits
+            const uint32_t tiles = (nout - 1) / per_tile / 8 + 1;  // on an XCD
             for (int mt = 1; mt <= (ft < 4 ? 4 : 3); ++mt) {
                 const uint32_t tb = (rows - 1) / (32u * (uint32_t)mt) + 1;
                 if ((tb > 1 && mt == 4) || 32 * mt >= (int)rows + 32) break;
-                const uint32_t per = (on_xcd * tb + 31) / 32;
+                if (splits > 1 && tiles * tb > 32) continue;
+                const uint32_t per = (tiles * (uint32_t)splits * tb + 31) / 32;
                 if (ft == 5 && per > 1) continue;
                 // workgroups that LDS holds at once: rings of up to 6 stages of 4 (FT + MT) KiB
                 const uint32_t resident = ft + mt == 2 ? 3 : ft + mt == 3 ? 2 : 1;
-                const double t = per * (stages * (0.050 * ft + 0.030 * mt + 0.0046 * ft * mt) + 0.27 * ft * mt) +
-                                 ((per - 1) / resident + 1) * (0.023 * stages + 0.69) + sums;
+                const double x = tb > 1 ? 0.0485 : 0.039;
+                const double t = per * (stages * (0.058 * ft + x * mt + 0.0175 * ft * mt) + 0.32 * ft * mt) +
+                                 ((per - 1) / resident + 1) * (0.010 * stages + 0.95) + sums;
                 if (!best.ft || t < least) best = TileCfg{ft, mt, splits}, least = t;
             }
         }
@@ -684,7 +691,7 @@ static bool tile_takes(int64_t M, int64_t N, int64_t K, bool gated) {
 // Of those, the products the kernel takes: not where the library measured faster
 // over 8973 products of 1 to 320 rows, N 8 to 151936, K 64 to 28672, weights from
 // HBM (hipBLASLt as torch 2.10 brings it, for gate_up pairs and silu_mul).  The
-// 8672 left are 0.57 of its time in the geometric mean, 131 of them over 1.03 and 52
+// 8672 left are 0.57 of its time in the geometric mean, 143 of them over 1.03 and 52
 // over 1.10 (1.47 at worst: its time jumps by as much between neighbouring shapes);
 // the 301 kept out 1.15.  Kept out, us, tile against library:
 //  - past 96 rows more than 24576 features, where the library's larger tiles
@@ -709,7 +716,7 @@ TileCfg tile_route(int64_t M, int64_t N, int64_t K, bool gated, size_t ws_bytes)
     if (deep && (K >= 4096 ? M <= 16 && mb < 52 : K >= 2048 && K < 3072 && M <= 8 && mb < 13)) return no;
     double us;
     const TileCfg c = tile_best(M, N, K, gated, ws_bytes, us);
-    if (deep && M > kDecodeRows && K >= 5120 && us > 10 && M * N * K < 420000000) return no;
+    if (deep && M > kDecodeRows && K >= 5120 && us > 12 && M * N * K < 420000000) return no;
     return c;
 }
 

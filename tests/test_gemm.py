@@ -290,6 +290,8 @@ def tile_form(M, N, K, gated=False, ws_bytes=64 << 20):
     (320, 1536, 8960, (3, 3, 4)),   # 22.5; (1, 2, 1) 40.3
     (77, 4096, 12288, (2, 3, 4)),   # 27.1, the fastest by either count
     (300, 4608, 3584, (3, 2, 1)),   # 22.6, likewise
+    (200, 3584, 18944, (4, 2, 2)),  # 63.4; (3, 3, 2) 72.8
+    (208, 3776, 23808, (4, 2, 2)),  # 82.8; (3, 3, 2) 101.3
     (77, 1024, 3072, (1, 1, 1)),    # a split saves 2 us on the GPU and costs a launch
 ])
 def test_tile_form_counts_workgroups_by_xcd(M, N, K, form):
@@ -423,7 +425,7 @@ def test_tile_gated_forms(gpu, orc, ft, mt):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,splits,bias", [
-    (33, 200, 5760, 2, True), (12, 400, 3840, 4, True), (37, 136, 3584, 8, True), (290, 72, 3840, 4, False),
+    (33, 200, 5760, 2, True), (12, 400, 3840, 4, True), (37, 136, 3584, 8, True), (290, 72, 4864, 4, False),
 ])
 def test_linear_tile_splits(gpu, orc, M, N, K, splits, bias):
     """Products whose K the LDS-tile kernel splits: the sums through the context's
